@@ -28,9 +28,9 @@ FLAGS = [
 ]
 
 
-# Per-file additions.  mmq.hip: keep MFMA accumulators in ordinary VGPRs, so
+# Per-file additions.  The MMQ files: keep MFMA accumulators in ordinary VGPRs, so
 # the per-element scaling reads them without v_accvgpr_read copies.
-FILE_FLAGS = {"mmq.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+FILE_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for f in ("mmq.hip", "mmq_planes.hip")}
 
 
 def _compile(src: Path) -> Path:

@@ -97,16 +97,35 @@ static bool mmq_supported(int ttype) {
          ttype == TT_IQ4_XS || ttype == TT_Q3_K || ttype == TT_Q2_K;
 }
 
-// The Exec mirror multiplies Q6_K weights by many tokens from their plane
-// image (built once per weight).  Measured on MI355X with the weights streamed
-// from HBM, [5120, 17408]: 48.8 / 51.9 / 53.1 / 64.7 / 76.3 / 124.6 us at 64 /
-// 96 / 128 / 192 / 256 / 512 tokens, against 49.0 / 77.8 / 78.7 / 160.9 /
-// 231.3 / 293.2 for the GGUF-row MMQ (the previous, row-major Q6_K image:
-// 54.0 / 59.6 / 61.2 / 82.0 / 106.9 / 205.9).  Up to 64 tokens the fragment
-// image (46.9 us at 64).  Q4_K stays on its fragment image: its MMQ image's
-// 3.9x larger weight bytes cost more than the scaling they save.
-bool mmq_image_preferred(const GemvArgs& g) {
-  return g.ttype == TT_Q6_K && g.tokens > 64 && mmq_image_bytes(g.ttype, g.rows, g.cols) > 0 && fast_ok(g);
+// The Exec mirror multiplies the super-block formats by a prompt's tokens from
+// their plane image (built once per weight, mmq_planes.hip).  Measured on
+// MI355X with the weights streamed from HBM, quantize and product together
+// (us), against the launches it replaces -- Q6_K its former plane-image kernel
+// on Q8_K rows, the others the tile MMQ on the GGUF rows:
+//
+//               tokens   [17408, 5120]            [2560, 9728]
+//   Q6_K     512 / 2048  116 / 381 vs 136 / 439   54 / 146 vs 60 / 168
+//   Q5_K      80 / 512    59 / 138 vs 100 / 244   37 / 59  vs 34 / 102
+//   Q5_K          2048         412 vs 859              153 vs 282
+//   Q3_K      37 / 512    32 / 83  vs 53 / 228    19 / 42  vs 25 / 126
+//   Q2_K      80 / 512    50 / 93  vs 82 / 226    24 / 47  vs 31 / 121
+//   IQ4_XS   130 / 512    73 / 122 vs 96 / 166    34 / 57  vs 60 / 92
+//   IQ3_XXS  130 / 512    67 / 118 vs 83 / 172    34 / 55  vs 62 / 92
+//   IQ3_S    130 / 512    69 / 118 vs 91 / 186    34 / 56  vs 68 / 105
+//
+// Below the thresholds the two-plane image's 2.06 bytes a weight cost more
+// than the tile MMQ's decode (IQ4_XS [17408, 5120] x 64 50 vs 39 us, Q2_K
+// [9728, 2560] x 64 19.1 vs 18.4); Q6_K up to 64 tokens reads its fragment
+// image.  Q4_K stays on its fragment image, a quarter of the bytes: 512 tokens
+// [17408, 5120] 125 us against 133 from its planes.
+bool planes_preferred(const GemvArgs& g) {
+  if (g.tokens > 65535 || planes_image_bytes(g.ttype, g.rows, g.cols) <= 0 || !fast_ok(g)) return false;
+  switch (g.ttype) {
+    case TT_Q6_K: case TT_Q5_K: case TT_Q2_K: return g.tokens > 64;
+    case TT_Q3_K: return g.tokens > 24;
+    case TT_IQ4_XS: case TT_IQ3_XXS: case TT_IQ3_S: return g.tokens > 128;
+    default: return false;
+  }
 }
 
 // Batches of a large Q6_K or Q4_K weight: the Exec mirror multiplies them

@@ -22,7 +22,7 @@
 namespace qhip {
 hipError_t dispatch_mul_mat(const GemvArgs& g, int path, void* work, long work_bytes, hipStream_t s);
 long mul_mat_work_bytes(const GemvArgs& g);
-bool mmq_image_preferred(const GemvArgs& g);
+bool planes_preferred(const GemvArgs& g);
 bool wd_image_preferred(const GemvArgs& g);
 }
 
@@ -261,7 +261,7 @@ static void* image_for(qhip_backend* be, const void* wdev, int ttype, int rows, 
   auto it = be->images.find(key);
   if (it != be->images.end()) return it->second.p;
   if (!be->images_on || capturing(be->stream)) return nullptr;
-  const long n = kind == kImgFrag ? qhip_wd_image_bytes(ttype, rows, cols) : qhip_mmq_image_bytes(ttype, rows, cols);
+  const long n = kind == kImgFrag ? qhip_wd_image_bytes(ttype, rows, cols) : planes_image_bytes(ttype, rows, cols);
   if (n <= 0 || over_budget(be, (size_t)n)) return nullptr;
   void* img = nullptr;
   hipError_t e = hipMalloc(&img, (size_t)n);
@@ -269,8 +269,10 @@ static void* image_for(qhip_backend* be, const void* wdev, int ttype, int rows, 
     *err = e;
     return nullptr;
   }
-  const int rc = kind == kImgFrag ? qhip_launch_wd_prepare(ttype, wdev, rows, cols, img, be->stream)
-                                  : qhip_launch_mmq_prepare(ttype, wdev, rows, cols, img, be->stream);
+  const int rc = kind == kImgFrag
+                     ? qhip_launch_wd_prepare(ttype, wdev, rows, cols, img, be->stream)
+                     : (int)launch_planes_prepare(ttype, wdev, qhip_weight_row_bytes(ttype, cols), rows, cols, img,
+                                                  be->stream);
   if (rc) {
     (void)hipFree(img);
     *err = (hipError_t)rc;
@@ -292,6 +294,8 @@ static size_t act_bytes_for(int cols, int k) {
 // its layout (gemv_image_layout; the other families are the activation
 // block sizes, 32 and 256)
 static constexpr int kFamSplit = 1 << 16;
+// memo family of the activation image the plane-image MMQ reads
+static constexpr int kFamMmq = 1 << 15;
 
 static hipError_t img_arena_alloc(qhip_backend* be, size_t bytes, uint8_t** out) {
   bytes = (bytes + kAlign - 1) / kAlign * kAlign;
@@ -431,6 +435,42 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
       if (ei != hipSuccess) return report("GEMV image", ei);
     }
   }
+  {
+    // a prompt: the MMQ from the weight's plane image, on the activation image
+    const GemvArgs gp{ttype, wdev, x, out, rows, cols, k, row_bytes, qhip_act_row_bytes(ttype, cols)};
+    if (planes_preferred(gp)) {
+      hipError_t e;
+      const void* img = image_for(be, wdev, ttype, rows, cols, kImgMmq, &e);
+      if (e != hipSuccess) return report("MMQ image", e);
+      if (img) {
+        const bool hm = be->memo_on && be->memo_src == x && be->memo_cols == cols && be->memo_k == k &&
+                        be->memo_fam == kFamMmq && be->act;
+        if (be->memo_on) (hm ? be->memo_hits : be->memo_misses)++;
+        if (!hm) {
+          e = ensure_act(be, (size_t)planes_act_bytes(cols, k));
+          if (e != hipSuccess) return report("activation scratch", e);
+          memo_clear(be);
+          e = launch_quantize_mmq_act(x, be->act, cols, k, be->stream);
+          if (e != hipSuccess) return report("quantize", e);
+          if (be->memo_on) {
+            be->memo_src = x;
+            be->memo_cols = cols;
+            be->memo_k = k;
+            be->memo_fam = kFamMmq;
+          }
+        }
+        // the split workspace is grown outside a capture only (under capture
+        // a launch that does not fit runs unsplit)
+        const long need = planes_work_bytes(rows, cols, k);
+        if (need > 0 && (size_t)need > be->skwork_cap && !capturing(be->stream)) {
+          e = ensure_skwork(be, (size_t)need);
+          if (e != hipSuccess && e != hipErrorOutOfMemory) return report("split-K workspace", e);
+        }
+        return report("matvec", launch_mmq_planes(ttype, img, be->act, out, rows, cols, k, be->skwork,
+                                                  (long)be->skwork_cap, be->stream));
+      }
+    }
+  }
   const bool hit = be->memo_on && be->memo_src == x && be->memo_cols == cols && be->memo_k == k &&
                    be->memo_fam == fam && be->act;
   if (be->memo_on) (hit ? be->memo_hits : be->memo_misses)++;
@@ -508,14 +548,6 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
     if (img)
       return report("matvec", (hipError_t)qhip_launch_mul_mat_wd_image(img, be->act, out, rows, cols, k, ttype, work,
                                                                         work_bytes, be->stream));
-  }
-  if (mmq_image_preferred(g)) {
-    // prefill of a Q6_K weight: MMQ from its image when there is one
-    void* img = image_for(be, wdev, ttype, rows, cols, kImgMmq, &e);
-    if (e != hipSuccess) return report("MMQ image", e);
-    if (img)
-      return report("matvec", (hipError_t)qhip_launch_mul_mat_image(img, be->act, out, rows, cols, k, ttype, 0, 0,
-                                                                     work, work_bytes, be->stream));
   }
   return report("matvec", dispatch_mul_mat(g, QHIP_PATH_AUTO, work, work_bytes, be->stream));
 }
@@ -704,7 +736,7 @@ int qhip_backend_prepare_linear(qhip_backend* be, const qhip_linear* w) {
   for (const int kind : {kImgFrag, kImgMmq}) {
     const GemvArgs g{w->ttype, w->dev, w->dev, nullptr, w->rows, w->cols, kind == kImgFrag ? 8 : 4096,
                      w->row_bytes, qhip_act_row_bytes(w->ttype, w->cols)};
-    if (!(kind == kImgFrag ? wd_image_preferred(g) : mmq_image_preferred(g))) continue;
+    if (!(kind == kImgFrag ? wd_image_preferred(g) : planes_preferred(g))) continue;
     if (capturing(be->stream)) return (int)hipErrorStreamCaptureUnsupported;
     hipError_t e;
     void* img = image_for(be, w->dev, w->ttype, w->rows, w->cols, kind, &e);

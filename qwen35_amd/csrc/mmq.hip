@@ -1224,14 +1224,14 @@ __global__ __launch_bounds__(256) void k_mmq_img(const uint8_t* __restrict__ IMG
 }
 
 long mmq_image_bytes(int ttype, int rows, int cols) {
-  if (ttype == TT_Q6_K) return bg_image_bytes_q6k(rows, cols);
+  if (ttype == TT_Q6_K) return planes_image_bytes(ttype, rows, cols);
   if (ttype != TT_Q4_K || rows < 0 || cols <= 0 || cols % 256) return -1;
   return (long)rows * (cols / 256) * (512 + img_hdr_bytes<TT_Q4_K>());
 }
 
 hipError_t launch_mmq_prepare(int ttype, const void* w, long row_bytes, int rows, int cols, void* img,
                               hipStream_t s) {
-  if (ttype == TT_Q6_K) return launch_bg_prepare_q6k(w, row_bytes, rows, cols, img, s);
+  if (ttype == TT_Q6_K) return launch_planes_prepare(ttype, w, row_bytes, rows, cols, img, s);
   if (ttype != TT_Q4_K) return hipErrorInvalidValue;
   const long nsb_total = (long)rows * (cols / 256);
   if (nsb_total <= 0) return hipSuccess;
@@ -2333,15 +2333,10 @@ static hipError_t launch_mmq_q8i(const GemvArgs& g, hipStream_t s) {
   return hipGetLastError();
 }
 
-// ---- Q6_K MMQ from the plane image (long prompts) ---------------------------------------
-// The plane image of a Q6_K weight holds p = sc (q6 - 32) for every value
-// (kernels256.c:200-212, :720-738: q6 from ql and qh, sc the 16-value
-// group's int8 scale) split exactly as p = 64 hi + lo (lo = p & 63, hi = p >> 6
-// >= -64), both planes in MFMA fragment order: per 32-row group and
-// super-block, 8 KB of hi fragments (sub-block s at 1024 s, lane L's 16 bytes
-// at 16 L: row L % 32, values 32 s + 16 (L / 32) ..+15), 8 KB of lo fragments,
-// then the 32 rows' f32 scales d -- 16,512 bytes per 32 rows and 256 values,
-// 2.5x the GGUF bytes.  Every weight load is one aligned, contiguous 1 KB.
+// ---- Q6_K MMQ from the plane image and Q8_K rows ----------------------------------------
+// The product of qhip_launch_mul_mat_image, whose activations are the
+// reference's Q8_K rows; the Exec mirror multiplies from the same plane image
+// (its layout: mmq_planes.hip) with an activation image instead.
 //
 // Tiles of 128 rows x TK = 32 NA tokens.  Within a workgroup of four waves,
 // wave w takes row group w and all TK tokens as NA 32 x 32 tiles, so each
@@ -2371,7 +2366,7 @@ static hipError_t launch_mmq_q8i(const GemvArgs& g, hipStream_t s) {
 // sliced tile is finished deterministically: each slice writes its partial
 // tile to the workspace, the last to arrive adds the P partials in slice
 // order and writes the outputs.
-constexpr int kBgQ6Grp = 16512;  // plane image bytes per 32-row group and super-block
+constexpr int kBgQ6Grp = 16512;  // plane image bytes per 32-row group and super-block (mmq_planes.hip)
 
 struct BgPlan {
   int ntt, nsb, ntiles, nwg;
@@ -2625,56 +2620,6 @@ __global__ __launch_bounds__(256, 2) void k_mmq_bg_q6k(const uint8_t* __restrict
     if (!more) break;
     cu = nu;
   }
-}
-
-// One thread per (32-row group, super-block, sub-block s, lane L): the 16
-// values 32 s + 16 (L / 32) .. +15 of row 32 group + L % 32 as both planes,
-// and for s = 0 the row's f32 scale.  Rows past the end: zeros.
-__global__ __launch_bounds__(256) void k_bg_prepare_q6k(const uint8_t* __restrict__ W, uint8_t* __restrict__ IMG,
-                                                         int rows, long row_bytes, int nsb, long nthreads) {
-  const long gid = (long)blockIdx.x * 256 + threadIdx.x;
-  if (gid >= nthreads) return;
-  const int Lq = (int)(gid & 63), s = (int)((gid >> 6) & 7);
-  const long gs = gid >> 9;  // group * nsb + sb
-  const long grp = gs / nsb;
-  const int sb = (int)(gs - grp * nsb);
-  const long row = grp * 32 + (Lq & 31);
-  const int e0 = 32 * s + 16 * (Lq >> 5);
-  uint32_t hi[4] = {0, 0, 0, 0}, lo[4] = {0, 0, 0, 0};
-  float d = 0.0f;
-  if (row < rows) {
-    const uint8_t* blk = W + row * row_bytes + 210L * sb;
-    const int sc = (int)(int8_t)blk[192 + (e0 >> 4)];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int e = e0 + i, h = e >> 7, q = (e & 127) >> 5, l = e & 31;
-      uint32_t lq = blk[64 * h + 32 * (q & 1) + l];
-      lq = q >= 2 ? (lq >> 4) : (lq & 15u);
-      const uint32_t hb = (blk[128 + 32 * h + l] >> (2 * q)) & 3u;
-      const int pv = sc * ((int)(lq | (hb << 4)) - 32);
-      hi[i >> 2] |= ((uint32_t)(pv >> 6) & 255u) << (8 * (i & 3));  // arithmetic shift: floor
-      lo[i >> 2] |= (uint32_t)(pv & 63) << (8 * (i & 3));
-    }
-    d = h2f((uint32_t)blk[208] | ((uint32_t)blk[209] << 8));
-  }
-  uint8_t* b = IMG + gs * kBgQ6Grp;
-  *(uint4*)(b + 1024 * s + 16 * Lq) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-  *(uint4*)(b + 8192 + 1024 * s + 16 * Lq) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-  if (s == 0 && Lq < 32) *(float*)(b + 16384 + 4 * Lq) = d;
-}
-
-long bg_image_bytes_q6k(int rows, int cols) {
-  if (rows < 0 || cols <= 0 || cols % 256) return -1;
-  return (long)((rows + 31) / 32) * (cols / 256) * kBgQ6Grp;
-}
-
-hipError_t launch_bg_prepare_q6k(const void* w, long row_bytes, int rows, int cols, void* img, hipStream_t s) {
-  if (bg_image_bytes_q6k(rows, cols) < 0) return hipErrorInvalidValue;
-  const long n = (long)((rows + 31) / 32) * (cols / 256) * 512;
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_bg_prepare_q6k, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (const uint8_t*)w,
-                     (uint8_t*)img, rows, row_bytes, cols / 256, n);
-  return hipGetLastError();
 }
 
 // Token tiles of the plane-image MMQ: 64 tokens up to 192, else 128.

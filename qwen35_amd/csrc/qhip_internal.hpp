@@ -81,10 +81,22 @@ hipError_t launch_mmq_prepare(int ttype, const void* w, long row_bytes, int rows
 // g.w = the image; bt x br tile (0 = default; splits K as launch_mmq); Q6_K
 // (the plane image) has one shape and ignores bt, br
 hipError_t launch_mmq_image(const GemvArgs& g, int bt, int br, void* work, long work_bytes, hipStream_t s);
-// Q6_K plane image and its MMQ (mmq.hip); the workspace: bg_work_bytes (0:
-// none needed), its first kSkCountBytes zero; nwg > 0 overrides the grid
-long bg_image_bytes_q6k(int rows, int cols);
-hipError_t launch_bg_prepare_q6k(const void* w, long row_bytes, int rows, int cols, void* img, hipStream_t s);
+// Plane image and activation image of the prompt MMQ (mmq_planes.hip): the
+// super-block formats, whose block integers are sums of scale * value.  The
+// workspace: planes_work_bytes (0: none needed), its first kSkCountBytes zero;
+// without it no tile is cut over K.
+bool planes_format(int ttype);
+long planes_image_bytes(int ttype, int rows, int cols);
+hipError_t launch_planes_prepare(int ttype, const void* w, long row_bytes, int rows, int cols, void* img,
+                                 hipStream_t s);
+long planes_act_bytes(int cols, int tokens);
+hipError_t launch_quantize_mmq_act(const float* x, void* out, int cols, int tokens, hipStream_t s);
+long planes_work_bytes(int rows, int cols, int tokens);
+hipError_t launch_mmq_planes(int ttype, const void* img, const void* xa, float* out, int rows, int cols, int tokens,
+                             void* work, long work_bytes, hipStream_t s);
+// The MMQ from Q6_K's plane image and Q8_K rows (mmq.hip); the workspace:
+// bg_work_bytes (0: none needed), its first kSkCountBytes zero; nwg > 0
+// overrides the grid
 long bg_work_bytes(const GemvArgs& g, int nwg);
 hipError_t launch_mmq_bg_q6k(const GemvArgs& g, void* work, long work_bytes, hipStream_t s, int nwg);
 // Q6_K fragment image (the GGUF bytes permuted for the few-token MMQ)

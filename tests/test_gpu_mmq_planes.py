@@ -1,0 +1,172 @@
+"""GPU: the prompt MMQ from plane and activation images, through the Exec
+mirror: every format and every switch of its dispatch (the token count it
+starts at, 64- against 128-token tiles, sliced and whole tiles) at row counts
+that are no multiple of a tile, against the oracle; exact block integers at
+unit scales and at the largest scales and values; the activation image byte
+for byte; a captured launch replayed; the activation memo across families."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import pyoracle as po
+from qwen35_amd import _lib, ops, synth
+from test_gpu_mmq import rel_l2, to_dev, unit_scale_act, unit_scale_weight
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-5
+# format: the token count the route starts at
+STARTS = {po.TT_Q6_K: 65, po.TT_Q5_K: 65, po.TT_Q2_K: 65, po.TT_Q3_K: 25, po.TT_IQ4_XS: 129, po.TT_IQ3_XXS: 129,
+          po.TT_IQ3_S: 129}
+
+
+@pytest.fixture
+def backend(gpu):
+    be = ops.Backend(0)
+    yield be
+    be.close()
+
+
+def product(be, tt, wd, rows, cols, x, images=True):
+    tokens = x.shape[0]
+    lin = be.wrap_linear(tt, rows, cols, wd)
+    be.set_mmq_images(images)
+    out = torch.full((tokens, rows), float("nan"), device=x.device)
+    be.matvec_batch_k(out, lin, x, tokens)
+    be.set_mmq_images(True)
+    placed = be.mem_placed()
+    be.free_linear(lin)
+    return out, placed - be.mem_placed()
+
+
+@pytest.mark.parametrize("tt", list(STARTS))
+def test_planes_match_oracle(gpu, oracle, backend, tt):
+    rows, cols = 333, 2048
+    w = synth.make_weight(tt, rows, cols, seed=41, tag=tt)
+    wd = to_dev(w, gpu)
+    for tokens in (STARTS[tt] - 1, STARTS[tt], 130, 256, 257, 300):
+        x = synth.make_act(cols, tokens, seed=42, tag=tokens)
+        xd = to_dev(x, gpu)
+        got, image = product(backend, tt, wd, rows, cols, xd)
+        assert rel_l2(got.cpu().numpy(), oracle.matvec(tt, w, x)) < TOL
+        if tt != po.TT_Q6_K:  # which has a fragment image too
+            assert (image > 0) == (tokens >= STARTS[tt])
+        again, _ = product(backend, tt, wd, rows, cols, xd)
+        assert torch.equal(got, again)  # the slices are added in a fixed order
+        plain, image = product(backend, tt, wd, rows, cols, xd, images=False)
+        assert image == 0 and rel_l2(plain.cpu().numpy(), got.cpu().numpy()) < 1e-6
+
+
+# 17408 x 256 rows and K of one super-block: whole rounds of tiles and nothing
+# to slice; 66 x 8192: a few tiles, sliced; 4224 x 2048: a full round of
+# 128-token tiles of 256 rows and a sliced remainder
+@pytest.mark.parametrize("tt", [po.TT_Q6_K, po.TT_Q3_K, po.TT_Q5_K])
+@pytest.mark.parametrize("rows,cols,tokens", [(17408, 256, 90), (66, 8192, 257), (4224, 2048, 2100)])
+def test_planes_grids(gpu, oracle, backend, tt, rows, cols, tokens):
+    w = synth.make_weight(tt, rows, cols, seed=43, tag=tt)
+    x = synth.make_act(cols, tokens, seed=44)
+    wd, xd = to_dev(w, gpu), to_dev(x, gpu)
+    got, _ = product(backend, tt, wd, rows, cols, xd)
+    pick = np.unique(np.linspace(0, rows - 1, 70).astype(int))
+    tpick = np.unique(np.linspace(0, tokens - 1, 60).astype(int))
+    want = oracle.matvec(tt, np.ascontiguousarray(w[pick]), np.ascontiguousarray(x[tpick]))
+    assert rel_l2(got.cpu().numpy()[np.ix_(tpick, pick)], want) < TOL
+    plain, _ = product(backend, tt, wd, rows, cols, xd, images=False)
+    assert rel_l2(plain.cpu().numpy(), got.cpu().numpy()) < 1e-6
+
+
+@pytest.mark.parametrize("tt", [po.TT_Q6_K, po.TT_Q5_K, po.TT_Q3_K, po.TT_Q2_K, po.TT_IQ4_XS])
+@pytest.mark.parametrize("tokens", [140, 270])
+def test_planes_integers_exact(gpu, oracle, backend, tt, tokens):
+    """d = dmin = 1 and activations of Q8_K scale 1: every output is the exact
+    integer sum of its row (one super-block, below 2^24)."""
+    rows, cols = 70, 256
+    w = unit_scale_weight(tt, rows, cols, seed=45)
+    x = unit_scale_act(cols, tokens, seed=46)
+    want = oracle.matvec(tt, w, x)
+    assert np.abs(want).max() < 2 ** 24 and np.array_equal(want, np.rint(want))
+    got, _ = product(backend, tt, to_dev(w, gpu), rows, cols, to_dev(x, gpu))
+    assert np.array_equal(got.cpu().numpy(), want)
+
+
+def test_planes_largest_values(gpu, oracle, backend):
+    """Q3_K's product -32 x -4 = 128 (held as -128) and Q6_K's -128 x -32 =
+    4096 in every place, activations +-127: the ends of the planes' range."""
+    cols, rows, tokens = 256, 64, 140
+    x = np.where(np.arange(cols) % 3 == 0, -127.0, 127.0).astype(np.float32)[None].repeat(tokens, 0)
+    w3 = np.zeros((rows, 110), np.uint8)  # scales 0 (-32), q2 0 and hmask 0 (-4)
+    w3[:, 108:110] = np.array([1.0], np.float16).view(np.uint8)
+    w6 = np.zeros((rows, 210), np.uint8)  # ql, qh 0 (-32)
+    w6[:, 192:208] = 0x80
+    w6[:, 208:210] = np.array([1.0], np.float16).view(np.uint8)
+    for tt, w in ((po.TT_Q3_K, w3), (po.TT_Q6_K, w6)):
+        got, _ = product(backend, tt, to_dev(w, gpu), rows, cols, to_dev(x, gpu))
+        assert np.array_equal(got.cpu().numpy(), oracle.matvec(tt, w, x))
+
+
+@pytest.mark.parametrize("shift", [0, 1])  # x 16-byte aligned, and 4 bytes past it
+def test_activation_image_bytes(gpu, oracle, shift):
+    """The image holds the Q8_K rows' bytes: quants 512 v + 16 t, sums as f16,
+    scales; tokens past the end are zeros."""
+    cols, tokens = 768, 45
+    x = synth.make_act(cols, tokens, seed=47)
+    x[3, 300] = np.nan
+    x[5, :256] = 0.0
+    buf = torch.empty(tokens * cols + 4, device=gpu)
+    xd = buf[shift:shift + tokens * cols].view(tokens, cols)
+    xd.copy_(to_dev(x, gpu))
+    dll = ctypes.CDLL(str(_lib.LIB_PATH))
+    quantize = dll["_ZN4qhip23launch_quantize_mmq_actEPKfPviiP12ihipStream_t"]
+    quantize.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
+    out = torch.empty(2 * 3 * 9344, dtype=torch.uint8, device=gpu)
+    assert quantize(xd.data_ptr(), out.data_ptr(), cols, tokens, torch.cuda.current_stream().cuda_stream) == 0
+    img = out.cpu().numpy().reshape(2, 3, 9344)
+    act = oracle.quantize_act(po.TT_Q6_K, x).reshape(tokens, 3, 292)
+    for tg in range(2):
+        n = min(32, tokens - 32 * tg)
+        a = act[32 * tg:32 * tg + n].transpose(1, 0, 2)  # [sb, token, byte]
+        q = img[tg, :, :8192].reshape(3, 16, 32, 16).transpose(0, 2, 1, 3).reshape(3, 32, 256)
+        assert np.array_equal(q[:, :n], a[:, :, 4:260]) and not q[:, n:].any()
+        s = img[tg, :, 8192:9216].copy().view(np.float16).reshape(3, 2, 4, 16, 4).transpose(0, 1, 3, 2, 4).reshape(3, 32, 16)
+        assert np.array_equal(s[:, :n], np.ascontiguousarray(a[:, :, 260:]).view(np.int16).astype(np.float16))
+        d = img[tg, :, 9216:].copy().view(np.float32)
+        assert np.array_equal(d[:, :n], np.ascontiguousarray(a[:, :, :4]).view(np.float32)[..., 0])
+
+
+def test_planes_captured_and_memo(gpu, oracle, backend):
+    """A captured launch replays on new activations; with the memo on, a second
+    product of the same x reuses the image, and a a product of another activation
+    family does not meet it."""
+    tt, rows, cols, tokens = po.TT_Q5_K, 300, 1024, 150
+    w = synth.make_weight(tt, rows, cols, seed=48)
+    lin = backend.wrap_linear(tt, rows, cols, to_dev(w, gpu))
+    assert backend.prepare_linear(lin) == 0
+    xs = [synth.make_act(cols, tokens, seed=49 + i) for i in range(3)]
+    x, out = to_dev(xs[0], gpu), torch.empty((tokens, rows), device=gpu)
+    side = torch.cuda.Stream()
+    backend.set_stream(side)
+    with torch.cuda.stream(side):
+        backend.matvec_batch_k(out, lin, x, tokens)  # scratch and workspace grow here
+    side.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        backend.matvec_batch_k(out, lin, x, tokens)
+    for xi in xs:
+        x.copy_(to_dev(xi, gpu))
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert rel_l2(out.cpu().numpy(), oracle.matvec(tt, w, xi)) < TOL
+    backend.set_stream(torch.cuda.current_stream())
+    backend.set_act_memo(True)
+    h0, m0 = backend.act_stats()
+    first, second, few = (torch.empty((tokens, rows), device=gpu) for _ in range(3))
+    backend.matvec_batch_k(first, lin, x, tokens)
+    backend.matvec_batch_k(second, lin, x, tokens)
+    backend.set_mmq_images(False)  # another weight without an image: its GGUF rows, on Q8_K rows
+    backend.matvec_batch_k(few, backend.wrap_linear(tt, rows, cols, to_dev(w, gpu).clone()), x, tokens)
+    backend.set_mmq_images(True)
+    assert torch.equal(first, second) and rel_l2(few.cpu().numpy(), first.cpu().numpy()) < 1e-6
+    h1, m1 = backend.act_stats()
+    assert (h1 - h0, m1 - m0) == (1, 2)
