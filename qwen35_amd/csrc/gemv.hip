@@ -314,20 +314,16 @@ __global__ __launch_bounds__(WGS) void k_gemv_q(const uint8_t* __restrict__ W, c
   // the first weight unit's: loads complete in order, so the quantize can
   // start as soon as x arrives instead of after the weights.
   constexpr int RX = 4;
-  constexpr int STEP = K32 ? WGS / 32 : WGS / 64;  // blocks per round
+  constexpr int STEP = K32 ? WGS / 8 : WGS / 64;  // blocks per round
   const bool out_q = XQ != nullptr && blockIdx.x == 0;
-  float xs[RX];
   float4 xf[RX];
+  const int qb = K32 ? threadIdx.x >> 3 : wv;                     // this lane's block of a round
+  const int qo = K32 ? 4 * (threadIdx.x & 7) : 4 * lane;          // and its four values
+  auto load_x = [&](int b) {
+    return b < nblk ? *(const float4*)(X + (K32 ? 32L : 256L) * b + qo) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  };
 #pragma unroll
-  for (int rd = 0; rd < RX; ++rd) {
-    if constexpr (K32) {
-      const int b = rd * STEP + (threadIdx.x >> 5);
-      xs[rd] = b < nblk ? X[32 * b + (threadIdx.x & 31)] : 0.0f;
-    } else {
-      const int b = rd * STEP + wv;
-      xf[rd] = b < nblk ? *(const float4*)(X + 256L * b + 4 * lane) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
-  }
+  for (int rd = 0; rd < RX; ++rd) xf[rd] = load_x(rd * STEP + qb);
 
   typename U::W wcur[NR];
   if (j < u_end) {
@@ -335,22 +331,19 @@ __global__ __launch_bounds__(WGS) void k_gemv_q(const uint8_t* __restrict__ W, c
     for (int k = 0; k < NR; ++k) wcur[k] = U::load_w(wrow[k], j);
   }
 
-  // one quantize round: block b from the value(s) v
-  auto quant32 = [&](int b, float v) {
-    const int i = threadIdx.x & 31;
-    const bool ok = b < nblk;
+  // one quantize round: block b from four values of each of its lanes
+  auto quant32 = [&](int b, float4 f) {
+    const float v[4] = {f.x, f.y, f.z, f.w};
     uint32_t hb;
-    const int q = quant_q8_0_lane(v, hb);
-    if (ok) {
-      qs[split_off(32 * b + i)] = (uint8_t)(int8_t)q;
-      if (i == 0) dsc[b] = h2f(hb);
+    const uint32_t packed = quant_q8_0_lane4(v, hb);
+    if (b < nblk) {
+      *(uint32_t*)(qs + split_off(32 * b + qo)) = packed;
+      if (qo == 0) dsc[b] = h2f(hb);
       if (out_q) {
         uint8_t* ob = XQ + 34L * b;
-        ob[2 + i] = (uint8_t)(int8_t)q;
-        if (i == 0) {
-          ob[0] = (uint8_t)hb;
-          ob[1] = (uint8_t)(hb >> 8);
-        }
+        *(uint16_t*)(ob + 2 + qo) = (uint16_t)packed;
+        *(uint16_t*)(ob + 4 + qo) = (uint16_t)(packed >> 16);
+        if (qo == 0) *(uint16_t*)ob = (uint16_t)hb;
       }
     }
   };
@@ -372,25 +365,17 @@ __global__ __launch_bounds__(WGS) void k_gemv_q(const uint8_t* __restrict__ W, c
       }
     }
   };
-  // K32: one value per thread, a 32-lane group per block; else a wave per
-  // 256-value block, four values per lane.  Rounds are uniform over the
-  // workgroup (every lane takes part in the shuffles).
+  // K32: eight lanes per block; else a wave per 256-value block; four values
+  // per lane.  Rounds are uniform over the workgroup (every lane takes part in
+  // the lane moves).
+  auto quant = [&](int b, float4 f) {
+    if constexpr (K32) quant32(b, f);
+    else quant256(b, f);
+  };
 #pragma unroll
-  for (int rd = 0; rd < RX; ++rd) {
-    if (rd * STEP < nblk) {
-      if constexpr (K32) quant32(rd * STEP + (threadIdx.x >> 5), xs[rd]);
-      else quant256(rd * STEP + wv, xf[rd]);
-    }
-  }
-  for (int b0 = RX * STEP; b0 < nblk; b0 += STEP) {
-    if constexpr (K32) {
-      const int b = b0 + (threadIdx.x >> 5);
-      quant32(b, b < nblk ? X[32 * b + (threadIdx.x & 31)] : 0.0f);
-    } else {
-      const int b = b0 + wv;
-      quant256(b, b < nblk ? *(const float4*)(X + 256L * b + 4 * lane) : make_float4(0.0f, 0.0f, 0.0f, 0.0f));
-    }
-  }
+  for (int rd = 0; rd < RX; ++rd)
+    if (rd * STEP < nblk) quant(rd * STEP + qb, xf[rd]);
+  for (int b0 = RX * STEP; b0 < nblk; b0 += STEP) quant(b0 + qb, load_x(b0 + qb));
   __syncthreads();
 
   float acc[NR];
@@ -999,7 +984,11 @@ static hipError_t launch_gemv_q_type(const GemvArgs& g, const float* x, void* xq
 bool gemv_fused_fits(int ttype, int cols) { return fused_lds_bytes(ttype, cols) <= kFusedMaxLds; }
 
 // Default fused shape: one row per lane and 1024-thread workgroups (16 waves
-// quantize the activation together, once per workgroup).  Lanes per row: the
+// quantize the activation together, once per workgroup); 512 threads for the
+// 32-value formats up to 2^23 weights, where the quantize is short and more
+// workgroups reach more CUs (Q8_0 [7168, 1024] 4.7 against 5.1 us, [2048,
+// 2048] 4.5 against 4.8, [1024, 3584] 5.0 against 5.2; at [2560, 6144] 1024
+// threads 7.8 against 8.7).  Lanes per row: the
 // candidate with the fewest wave-steps (waves x units per lane) among those
 // whose grid has at least 192 workgroups (three quarters of the CUs), ties to
 // the smaller team; if none fills the GPU, the largest grid.  Swept on MI355X
@@ -1012,6 +1001,7 @@ bool gemv_fused_fits(int ttype, int cols) { return fused_lds_bytes(ttype, cols) 
 // 9.10.
 static void fused_default_shape(const GemvArgs& g, int& team, int& nr, int& wgs) {
   static const int kCand[] = {8, 10, 16, 20, 32, 40, 64};
+  wgs = act32(g.ttype) && (long)g.rows * g.cols <= (1L << 23) ? 512 : 1024;
   const long upr = g.cols / 64;
   int best = -1;
   long best_w = 0, best_grid = 0;
@@ -1019,7 +1009,7 @@ static void fused_default_shape(const GemvArgs& g, int& team, int& nr, int& wgs)
   for (int t : kCand) {
     const long tpw = 64 / t;
     const long waves = (g.rows + tpw - 1) / tpw;
-    const long grid = (waves + 15) / 16;
+    const long grid = (waves + wgs / 64 - 1) / (wgs / 64);
     const long w = waves * ((upr + t - 1) / t);
     const bool full = grid >= 192;
     bool take;
@@ -1036,23 +1026,25 @@ static void fused_default_shape(const GemvArgs& g, int& team, int& nr, int& wgs)
   }
   team = best;
   nr = 1;
-  wgs = 1024;
 }
 
 // Fused quantize + GEMV against separate quantize and GEMV launches, measured
 // on MI355X with the default shapes: the fused launch wins for rows up to
-// 32768 at widths up to 4096 (Q4_K [19456, 2560] 9.4 vs 10.7 us, Q8_0 [6144,
-// 1024] 5.0 vs 6.2 us) and loses on long rows, where every workgroup would
-// quantize a long activation (Q6_K [2560, 9728] 12.4 vs 10.4 us, Q4_K
-// [17408, 5120] 14.9 vs 14.2 us).  The 32-value formats' separate GEMV takes
-// multi-row shapes the fused launch does not, and wins on larger matrices:
-// Q8_0 from width 4096 ([12288, 4096] 19.2 vs 22.1 us; [32768, 2560] fused
-// 21.0 vs 27.9), the 4-bit ones from 2^24 weights (Q4_0 [19456, 2560] 10.5
-// vs 11.9 us, IQ4_NL 11.8 vs 13.7; [6144, 1024] fused 4.7 vs 6.8).
+// 32768 at widths up to 4096 (Q4_K [19456, 2560] 9.4 vs 10.7 us) and loses on
+// long rows, where every workgroup would quantize a long activation (Q6_K
+// [2560, 9728] 12.4 vs 10.4 us, Q4_K [17408, 5120] 14.9 vs 14.2 us).  The
+// 32-value formats, since eight lanes share a block (four values a lane) in
+// the fused quantize (launches captured in a graph, weights streamed from
+// HBM): Q8_0 wins to width 6144 ([1024, 3584] 5.0 vs 7.2 us, [2560, 6144] 8.1
+// vs 10.3, [8192, 4096] 10.5 vs 14.1, [19456, 2560] 16.3 vs 18.7; [5120, 8192]
+// 16.5 vs 16.8 from split-K 13.3), the 4-bit ones to width 4096 below 2^26
+// weights (IQ4_NL [9728, 2560] 8.1 vs 9.7, [19456, 2560] 12.0 vs 12.8; Q4_1
+// [8192, 4096] 7.8 vs 8.9; [17408, 5120] 17.7 vs 15.2).
 bool gemv_fused_preferred(const GemvArgs& g) {
-  if (g.tokens != 1 || !gemv_fused_fits(g.ttype, g.cols) || g.cols > 4096 || g.rows > 32768) return false;
-  if (g.ttype == TT_Q8_0) return g.cols <= 2560;
-  if (act32(g.ttype)) return (long)g.rows * g.cols <= (1L << 24);
+  if (g.tokens != 1 || !gemv_fused_fits(g.ttype, g.cols) || g.rows > 32768) return false;
+  if (g.ttype == TT_Q8_0) return g.cols <= 6144;
+  if (g.cols > 4096) return false;
+  if (act32(g.ttype)) return (long)g.rows * g.cols < (1L << 26);
   return true;
 }
 

@@ -335,16 +335,17 @@ static hipError_t launch_img_tt(const GemvArgs& g, int T, int P, int nr, hipStre
 }
 
 // Quantize + image GEMV against the GGUF-layout launches (one token),
-// measured on MI355X (IQ4_NL, weights rotated past the Infinity Cache; GEMV
-// alone, then quantize + GEMV against the one-launch fused form): [248320,
-// 2560] 62.8 vs 72.6 us, 64.9 vs 74.7 (fused 79.1); [17408, 5120] 12.2 vs
-// 15.3; [19456, 2560] 8.2 vs 9.4, 10.6 vs 11.9 (fused 13.2); [8192, 4096]
-// 5.5 vs 7.0; [4096, 4096] 4.0 vs 4.8, 7.5 vs 7.8 (fused 8.1); [12288,
-// 2048] 4.8 vs 7.6; Q4_0 alike.  Below 2^23 weights the fused launch wins
-// ([6144, 1024]: fused 5.1 us, quantize + image GEMV 7.2).
+// measured on MI355X (weights rotated past the Infinity Cache; GEMV alone, then
+// quantize + GEMV against the one-launch fused form): IQ4_NL [248320, 2560]
+// 62.8 vs 72.6 us, 64.9 vs 74.7 (fused 79.1); [19456, 2560] 10.9 vs 12.8
+// (fused 12.0), Q8_0 14.4 vs 18.7 (16.3); at [8192, 4096] the two meet (IQ4_NL
+// 8.9 / fused 9.0, Q8_0 11.2 / 10.5, Q4_0 8.7 / 8.1).  Below 2^25 weights the
+// fused launch wins (Q8_0 [9728, 2560] 9.3 us against 10.0 from the image,
+// IQ4_NL [4096, 4096] 6.2 against 7.2, [6144, 1024] 4.4 against 5.6); rows too
+// wide for it read the image from 2^23.
 bool gemv_image_preferred(const GemvArgs& g) {
   return g.tokens == 1 && gemv_image_format(g.ttype) && gemv_image_width(g.cols) &&
-         (long)g.rows * g.cols > (1L << 23);
+         (long)g.rows * g.cols > (1L << 23) && (!gemv_fused_preferred(g) || (long)g.rows * g.cols >= (1L << 25));
 }
 
 // ---- K-quant GEMV image (Q4_K, Q6_K) --------------------------------------------

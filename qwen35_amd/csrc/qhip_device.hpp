@@ -100,16 +100,52 @@ __device__ __forceinline__ int trunc_i32_x86(float v) {
   return (v > -2147483904.0f && v < 2147483648.0f) ? (int)v : (int)0x80000000u;
 }
 
+// ---- lane moves -------------------------------------------------------------------
+// v of another lane by DPP (VALU lane moves: a few cycles each, against an LDS
+// round trip per step for ds_bpermute); 0 where there is no source lane or its
+// row is masked out.
+template <int CTRL, int ROW_MASK = 0xF>
+__device__ __forceinline__ float dpp_f32(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROW_MASK, 0xF, false));
+}
+// Maximum of a >= 0 over each 32-lane half of the wave, in every lane of it:
+// quads, half-rows and rows of 16 (quad_perm, mirrors), then rows 0 / 2 into
+// rows 1 / 3, whose last lanes hold the halves' maxima.
+__device__ __forceinline__ float half_max(float a) {
+  a = fmaxf(a, dpp_f32<0xB1>(a));        // quad_perm [1, 0, 3, 2]
+  a = fmaxf(a, dpp_f32<0x4E>(a));        // quad_perm [2, 3, 0, 1]
+  a = fmaxf(a, dpp_f32<0x141>(a));       // row_half_mirror
+  a = fmaxf(a, dpp_f32<0x140>(a));       // row_mirror
+  a = fmaxf(a, dpp_f32<0x142, 0xA>(a));  // row_bcast:15 into rows 1 and 3
+  const float lo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(a), 31));
+  const float hi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(a), 63));
+  return (threadIdx.x & 32) ? hi : lo;
+}
+// The same over the whole wave.
+__device__ __forceinline__ float wave_max(float a) {
+  a = fmaxf(a, dpp_f32<0xB1>(a));
+  a = fmaxf(a, dpp_f32<0x4E>(a));
+  a = fmaxf(a, dpp_f32<0x141>(a));
+  a = fmaxf(a, dpp_f32<0x140>(a));
+  a = fmaxf(a, dpp_f32<0x142, 0xA>(a));
+  a = fmaxf(a, dpp_f32<0x143, 0xC>(a));  // row_bcast:31 into rows 2 and 3
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(a), 63));
+}
+__device__ __forceinline__ int quad_sum(int s) {
+  s += __builtin_amdgcn_update_dpp(0, s, 0xB1, 0xF, 0xF, false);
+  s += __builtin_amdgcn_update_dpp(0, s, 0x4E, 0xF, 0xF, false);
+  return s;
+}
+
 // ---- activation quantizers, one block per lane group -------------------------------
 // Q8_0 (src/kernels/x86/kernels32.c:1064-1087): lane i of a 32-lane group holds
 // value i of the block.  Returns the lane's quantized value; `hbits` gets the
-// block's f16 scale bits.  Every lane of the group must call it (shuffles).
+// block's f16 scale bits.  Every lane of the group must call it (lane moves).
 __device__ __forceinline__ int quant_q8_0_lane(float v, uint32_t& hbits) {
   // |v| with the reference's "if (a > amax)" NaN handling: NaN never wins.
   float a = v < 0.0f ? -v : v;
   a = a > 0.0f ? a : 0.0f;
-#pragma unroll
-  for (int off = 16; off > 0; off >>= 1) a = fmaxf(a, __shfl_xor(a, off, 32));
+  a = half_max(a);
   const float scale = a > 0.0f ? a / 127.0f : 1.0f;
   const float inv = a > 0.0f ? 1.0f / scale : 0.0f;
   const float sv = v * inv;
@@ -119,6 +155,35 @@ __device__ __forceinline__ int quant_q8_0_lane(float v, uint32_t& hbits) {
   q = q < -128 ? -128 : q;
   hbits = f32_to_f16_bits(scale);
   return q;
+}
+
+// Q8_0 with four values per lane, eight consecutive lanes per block (lane 8 g
+// + i: values 4 i ..+3): the same bytes, packed (byte k = value 4 i + k).
+__device__ __forceinline__ uint32_t quant_q8_0_lane4(const float* v, uint32_t& hbits) {
+  float a = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float e = v[i] < 0.0f ? -v[i] : v[i];
+    e = e > 0.0f ? e : 0.0f;
+    a = fmaxf(a, e);
+  }
+  a = fmaxf(a, dpp_f32<0xB1>(a));   // quad_perm [1, 0, 3, 2]
+  a = fmaxf(a, dpp_f32<0x4E>(a));   // quad_perm [2, 3, 0, 1]
+  a = fmaxf(a, dpp_f32<0x141>(a));  // row_half_mirror: the eight lanes
+  const float scale = a > 0.0f ? a / 127.0f : 1.0f;
+  const float inv = a > 0.0f ? 1.0f / scale : 0.0f;
+  uint32_t packed = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float sv = v[i] * inv;
+    const float r = sv + (sv >= 0.0f ? 0.5f : -0.5f);
+    int q = trunc_i32_x86(r);
+    q = q > 127 ? 127 : q;
+    q = q < -128 ? -128 : q;
+    packed |= ((uint32_t)q & 0xFFu) << (8 * i);
+  }
+  hbits = f32_to_f16_bits(scale);
+  return packed;
 }
 
 // Q8_K (src/kernels/x86/kernels256.c:865-896): lane l of a wave holds values
@@ -133,8 +198,7 @@ __device__ __forceinline__ uint32_t quant_q8_K_lane(const float* v, int& gsum, f
     e = e > 0.0f ? e : 0.0f;
     a = fmaxf(a, e);
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) a = fmaxf(a, __shfl_xor(a, off, 64));
+  a = wave_max(a);
   scale = a > 0.0f ? a / 127.0f : 1.0f;
   const float inv = a > 0.0f ? 1.0f / scale : 0.0f;
   uint32_t packed = 0;
@@ -149,24 +213,16 @@ __device__ __forceinline__ uint32_t quant_q8_K_lane(const float* v, int& gsum, f
     packed |= ((uint32_t)q & 0xFFu) << (8 * i);
     s += q;
   }
-  s += __shfl_xor(s, 1, 64);
-  s += __shfl_xor(s, 2, 64);
-  gsum = s;
+  gsum = quad_sum(s);
   return packed;
 }
 
 // ---- wave reductions --------------------------------------------------------------
-// Sum of v over the 64 lanes of a wave, in lane 63, by DPP (VALU lane moves:
-// a few cycles each, against an LDS round trip per step for ds_bpermute).
-// Adjacent lanes and lane pairs within quads (quad_perm), then the mirrored
+// Sum of v over the 64 lanes of a wave, in lane 63, by DPP.  Adjacent lanes and lane pairs within quads (quad_perm), then the mirrored
 // half-rows and rows give every lane of a 16-lane row the row's sum;
 // row_bcast:15 adds row 0's sum into row 1 and row 2's into row 3,
 // row_bcast:31 then adds rows 0 + 1 into rows 2 and 3.  The order of the
 // additions is fixed, so the result is deterministic.
-template <int CTRL, int ROW_MASK = 0xF>
-__device__ __forceinline__ float dpp_f32(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROW_MASK, 0xF, false));
-}
 __device__ __forceinline__ float wave_sum_to_lane63(float v) {
   v += dpp_f32<0xB1>(v);         // quad_perm [1, 0, 3, 2]
   v += dpp_f32<0x4E>(v);         // quad_perm [2, 3, 0, 1]
