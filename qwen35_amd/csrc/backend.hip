@@ -81,7 +81,7 @@ struct qhip_backend {
   struct GImage {
     uint8_t* img;
     int ttype, rows, cols;
-    long row_bytes;
+    long row_bytes, img_row_bytes;
   };
   std::map<const uint8_t*, GImage> gimages;
   struct Chunk2 { uint8_t* base; size_t size, used; };
@@ -337,13 +337,13 @@ static uint8_t* gimage_lookup(const qhip_backend* be, const void* wdev, int ttyp
     if (g.ttype != ttype || g.cols != cols || g.row_bytes != row_bytes) return nullptr;
     const long off = (long)(p - it->first);
     if (off % row_bytes || off / row_bytes >= g.rows) return nullptr;
-    uint8_t* ip = g.img + off;
+    uint8_t* ip = g.img + off / row_bytes * g.img_row_bytes;
     if (first == nullptr) first = ip;
     else if (ip != expect) return nullptr;
     const long take = need < g.rows - off / row_bytes ? need : g.rows - off / row_bytes;
     need -= take;
     p += take * row_bytes;
-    expect = ip + take * row_bytes;
+    expect = ip + take * g.img_row_bytes;
   }
   return first;
 }
@@ -356,7 +356,8 @@ static uint8_t* gimage_for(qhip_backend* be, const void* wdev, int ttype, int ro
   *err = hipSuccess;
   if (uint8_t* hit = gimage_lookup(be, wdev, ttype, rows, cols, row_bytes)) return hit;
   if (!be->gemv_images_on || capturing(be->stream)) return nullptr;
-  const long n = qhip_gemv_image_bytes(ttype, rows, cols);
+  const long irb = gemv_image_row_bytes(ttype, cols, row_bytes);
+  const long n = gemv_kimage_own(ttype) ? irb * rows : qhip_gemv_image_bytes(ttype, rows, cols);
   if (n <= 0 || over_budget(be, (size_t)n)) return nullptr;
   uint8_t* img = nullptr;
   hipError_t e = img_arena_alloc(be, (size_t)n, &img);
@@ -364,12 +365,14 @@ static uint8_t* gimage_for(qhip_backend* be, const void* wdev, int ttype, int ro
     if (e != hipErrorOutOfMemory) *err = e;
     return nullptr;
   }
-  const int rc = qhip_launch_gemv_prepare(ttype, wdev, rows, cols, img, be->stream);
+  const int rc = gemv_kimage_own(ttype)
+                     ? (int)launch_kimage_prepare(ttype, wdev, row_bytes, rows, cols, img, be->stream)
+                     : qhip_launch_gemv_prepare(ttype, wdev, rows, cols, img, be->stream);
   if (rc) {
     *err = (hipError_t)rc;
     return nullptr;
   }
-  be->gimages[(const uint8_t*)wdev] = qhip_backend::GImage{img, ttype, rows, cols, row_bytes};
+  be->gimages[(const uint8_t*)wdev] = qhip_backend::GImage{img, ttype, rows, cols, row_bytes, irb};
   return img;
 }
 
@@ -423,9 +426,8 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
       }
     }
   }
-  // Q6_K at one token, quantized separately: the weight's K-quant GEMV image
-  // (the same GEMV launch as the GGUF rows, reading the image), in place of
-  // the one-launch split-K form
+  // Q6_K, Q2_K, Q3_K and Q5_K at one token, quantized separately: the GEMV
+  // from the weight's K-quant image, in place of the one-launch forms
   uint8_t* kimg = nullptr;
   if (k == 1 && be->gemv_images_on) {
     const GemvArgs gk{ttype, wdev, x, out, rows, cols, 1, row_bytes, qhip_act_row_bytes(ttype, cols)};
@@ -529,6 +531,7 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
   if (kimg) {
     GemvArgs gi = g;
     gi.w = kimg;
+    gi.row_bytes = gemv_image_row_bytes(ttype, cols, row_bytes);
     gi.kimg = true;
     return report("matvec", launch_gemv(gi, 0, 0, 0, be->stream));
   }

@@ -28,7 +28,7 @@ __global__ __launch_bounds__(64 * WPB) void k_gemv(const uint8_t* __restrict__ W
                                                const uint8_t* __restrict__ XQ,
                                                float* __restrict__ Y, int rows, long row_bytes,
                                                long act_bytes, int upr, int team, int tokens) {
-  using U = Unit<TT>;
+  using U = typename UnitOf<TT, IMG>::type;
   grid_prologue<TT>();
   const int lane = threadIdx.x & 63;
   const int tpw = 64 / team;                       // teams per wave
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256) void k_gemv_mw(const uint8_t* __restrict__ W,
                                                   const uint8_t* __restrict__ XQ,
                                                   float* __restrict__ Y, int rows, long row_bytes,
                                                   int upr) {
-  using U = Unit<TT>;
+  using U = typename UnitOf<TT, IMG>::type;
   grid_prologue<TT>();
   constexpr int TPB = 4 / WV;  // teams per workgroup
   __shared__ float part[4][NR];
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256) void k_gemv_mw(const uint8_t* __restrict__ W,
 template <int TT, int NR, int WV, int A, bool IMG = false>
 __global__ __launch_bounds__(256) void k_gemv_bal(const uint8_t* __restrict__ W, const uint8_t* __restrict__ XQ,
                                                    float* __restrict__ Y, int rows, long row_bytes, int upr) {
-  using U = Unit<TT>;
+  using U = typename UnitOf<TT, IMG>::type;
   constexpr int TPB = 4 / WV;  // teams per workgroup
   __shared__ float part[4][NR];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -686,11 +686,14 @@ int gemv_pick_team(int rows, int cols, int target_waves) {
 // 2-token and a 1-token pass (Q4_K [17408, 5120]).
 int gemv_pick_nt(int tokens) { return tokens > 4 ? 8 : tokens > 2 ? 4 : tokens > 1 ? 2 : 1; }
 
-// the two formats with a K-quant GEMV image (g.kimg)
+// the formats with a K-quant GEMV image (g.kimg)
 template <class F>
 static hipError_t dispatch_kimg(int ttype, F&& f) {
   if (ttype == TT_Q4_K) return f(std::integral_constant<int, TT_Q4_K>{});
   if (ttype == TT_Q6_K) return f(std::integral_constant<int, TT_Q6_K>{});
+  if (ttype == TT_Q2_K) return f(std::integral_constant<int, TT_Q2_K>{});
+  if (ttype == TT_Q3_K) return f(std::integral_constant<int, TT_Q3_K>{});
+  if (ttype == TT_Q5_K) return f(std::integral_constant<int, TT_Q5_K>{});
   return hipErrorInvalidValue;
 }
 
@@ -771,6 +774,16 @@ static hipError_t launch_gemv_type(const GemvArgs& g, int team, int nt, int nr, 
 // one row per 20-lane team at width 2560 (9.3 vs 10.1 us), two from 4096.
 static void default_shape(const GemvArgs& g, int& team, int& nr) {
   const int upr = g.cols / 64;
+  // the images of Q2_K, Q3_K and Q5_K: two-wave teams of two rows, also where
+  // a row has fewer units than lanes (Q3_K [6144, 2560] 4.6 us against 5.2
+  // with 20 lanes), and four-wave teams past 128 units ([2560, 9728] 5.4
+  // against 6.3); Q5_K with four rows at 64 < units <= 128 ([17408, 5120] 14.9
+  // against 15.6)
+  if (g.kimg && kimage_own(g.ttype)) {
+    team = upr > 128 ? 256 : 128;
+    nr = g.ttype == TT_Q5_K && upr > 64 && upr <= 128 && g.rows >= 8192 ? 4 : 2;
+    return;
+  }
   const bool nib32 = g.ttype == TT_Q4_0 || g.ttype == TT_Q4_1 || g.ttype == TT_IQ4_NL;
   // long rows: teams of whole waves (k_gemv_mw), several rows per team (the
   // Q6_K image two: [5120, 17408] 28.2 us with four against 18.1 from the
@@ -842,9 +855,27 @@ static hipError_t launch_gemv_multiwave(const GemvArgs& g, int nr, int wv, hipSt
 // against 6.1: half the waves in flight), and so do the GGUF rows, whose
 // misaligned 210-byte super-blocks lose with every load at once ([5120,
 // 17408] 21.0 against 19.0 us, [4096, 12288] 12.2 against 11.1).
+// The images of Q2_K, Q3_K and Q5_K: one wave of four rows where a = 1 and
+// 0 < b <= 16, of two otherwise, from 8192 rows (Q3_K [34816, 5120] 20.2 us
+// against 23.3 with two-wave teams, [14336, 4096] 7.9 against 8.8; Q5_K only
+// at b = 0, [14336, 4096] 9.9 against 10.2, as [17408, 5120] is 15.7 against
+// 14.9), and four waves of four rows where a = 4 (Q2_K [5120, 17408] 10.8
+// against 11.6; Q3_K 13.4 / 13.5, Q5_K 16.7 / 16.5).
 static bool bal_shape(const GemvArgs& g, int& nr, int& wv) {
-  if (!g.kimg || g.ttype != TT_Q6_K || g.tokens != 1 || g.rows < 4096 || g.cols % 256) return false;
+  if (!g.kimg || g.ttype == TT_Q4_K || g.tokens != 1 || g.rows < 4096 || g.cols % 256) return false;
   const int upr = g.cols / 64, a = upr / 64, b = upr % 64;
+  if (kimage_own(g.ttype)) {
+    if (a == 1 && g.rows >= 8192 && !(g.ttype == TT_Q5_K && b > 0)) {
+      nr = b > 0 && b <= 16 ? 4 : 2;
+      wv = 1;
+    } else if (a == 4) {
+      nr = 4;
+      wv = 4;
+    } else {
+      return false;
+    }
+    return nr * b <= 64 * wv;
+  }
   if (a == 1) {
     nr = 2;
     wv = 1;
@@ -870,16 +901,24 @@ static hipError_t launch_gemv_bal_t(const GemvArgs& g, hipStream_t s) {
 }
 
 static hipError_t launch_gemv_bal(const GemvArgs& g, int nr, int wv, hipStream_t s) {
-  if (g.ttype != TT_Q6_K || !g.kimg) return hipErrorInvalidValue;
-  if (wv == 1 && nr == 2) return launch_gemv_bal_t<TT_Q6_K, 2, 1, true>(g, s);
-  if (wv == 4 && nr == 2) return launch_gemv_bal_t<TT_Q6_K, 2, 4, true>(g, s);
-  if (wv == 4 && nr == 4) return launch_gemv_bal_t<TT_Q6_K, 4, 4, true>(g, s);
-  return hipErrorInvalidValue;
+  if (!g.kimg || g.ttype == TT_Q4_K) return hipErrorInvalidValue;
+  return dispatch_kimg(g.ttype, [&](auto tt) -> hipError_t {
+    constexpr int T = decltype(tt)::value;
+    if (wv == 1 && nr == 2) return launch_gemv_bal_t<T, 2, 1, true>(g, s);
+    if constexpr (kimage_own(T)) {
+      if (wv == 1 && nr == 4) return launch_gemv_bal_t<T, 4, 1, true>(g, s);
+    } else {
+      if (wv == 4 && nr == 2) return launch_gemv_bal_t<T, 2, 4, true>(g, s);
+    }
+    if (wv == 4 && nr == 4) return launch_gemv_bal_t<T, 4, 4, true>(g, s);
+    return hipErrorInvalidValue;
+  });
 }
 
 hipError_t launch_gemv(const GemvArgs& g, int team, int nt, int nr, hipStream_t s) {
   if (g.rows <= 0 || g.tokens <= 0) return hipSuccess;
-  if (g.kimg && (g.tokens != 1 || !kimage_format(g.ttype) || g.cols % 256)) return hipErrorInvalidValue;
+  if (g.kimg && (g.tokens != 1 || !(kimage_format(g.ttype) || kimage_own(g.ttype)) || g.cols % 256))
+    return hipErrorInvalidValue;
   if (team <= 0 && nr <= 0 && g.tokens == 1) {
     int bwv = 0;
     if (bal_shape(g, nr, bwv)) return launch_gemv_bal(g, nr, bwv, s);
@@ -904,12 +943,14 @@ hipError_t launch_gemv(const GemvArgs& g, int team, int nt, int nr, hipStream_t 
   if (g.kimg) {
     return dispatch_kimg(g.ttype, [&](auto tt) -> hipError_t {
       constexpr int T = decltype(tt)::value;
-      switch (nr) {
-        case 1: return launch_gemv_t<T, 1, 1, true>(g, team, s);
-        case 2: return launch_gemv_t<T, 1, 2, true>(g, team, s);
-        case 4: return launch_gemv_t<T, 1, 4, true>(g, team, s);
-        default: return hipErrorInvalidValue;
+      if constexpr (kimage_format(T)) {
+        switch (nr) {
+          case 1: return launch_gemv_t<T, 1, 1, true>(g, team, s);
+          case 2: return launch_gemv_t<T, 1, 2, true>(g, team, s);
+          case 4: return launch_gemv_t<T, 1, 4, true>(g, team, s);
+        }
       }
+      return hipErrorInvalidValue;  // the others' default shapes are whole waves
     });
   }
   return dispatch_type(g.ttype, [&](auto tt) { return launch_gemv_type<decltype(tt)::value>(g, team, nt, nr, s); });
@@ -1149,8 +1190,23 @@ bool gemv_splitk_preferred(const GemvArgs& g) {
 // [5120, 17408] 16.5), also instead of the split-K form: the config-2 decode
 // step (its Q6_K down projection [2560, 9728]) 17.8 against 19.2 us,
 // [5120, 17408] 18.4 against 18.3.
+//
+// The images that hold each unit's own bits (Q2_K, Q3_K, Q5_K: ImgUnit), GEMV
+// launch alone against the GGUF rows: Q3_K [34816, 5120] 20.2 against 35.8 us
+// (2.1 to 3.9 TB/s), [17408, 5120] 12.5 / 19.8, [5120, 17408] 13.4 / 22.2,
+// [2560, 9728] 5.4 / 10.0, [19456, 2560] 9.9 / 14.6; Q2_K [17408, 5120] 10.6 /
+// 11.9, [5120, 17408] 10.8 / 16.6, [2560, 9728] 4.7 / 6.9; Q5_K [17408, 5120]
+// 14.9 / 17.0, [5120, 17408] 16.5 / 20.8, [2560, 9728] 6.2 / 8.8.  With the
+// quantizer's 2.3 us Q2_K and Q5_K win wherever the one-launch form is not
+// preferred ([8192, 8192] Q2_K 9.7 against 9.9, Q5_K 13.9 / 14.8; against the
+// split-K form [2560, 9728] 7.0 / 8.9 and 8.5 / 10.0, [5120, 17408] 13.3 / 13.3
+// and 18.7 / 18.5) and lose where it is (Q2_K [19456, 2560] 10.5 / 8.9, Q5_K
+// [4096, 4096] 7.2 / 6.7).  Q3_K, whose GGUF unit is the dearest, wins there
+// too ([19456, 2560] 12.2 / 15.9, [4096, 4096] 6.5 / 7.3, [2560, 4096] 5.9 /
+// 6.4), so it takes the image from 2^23 weights.
 bool gemv_kimage_preferred(const GemvArgs& g) {
-  return g.tokens == 1 && g.ttype == TT_Q6_K && g.cols % 256 == 0 && !gemv_fused_preferred(g);
+  if (g.tokens != 1 || g.cols % 256 || !(g.ttype == TT_Q6_K || kimage_own(g.ttype))) return false;
+  return !gemv_fused_preferred(g) || (g.ttype == TT_Q3_K && (long)g.rows * g.cols > (1L << 23));
 }
 
 hipError_t launch_gemv_splitk(const GemvArgs& g, const float* x, void* xq_out, int team, int nr, int slice,

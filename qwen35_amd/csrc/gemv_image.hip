@@ -356,6 +356,8 @@ bool gemv_image_preferred(const GemvArgs& g) {
 // The GEMV, fused and split-K launchers of gemv.hip read it when g.kimg, with
 // the activation in the reference Q8_K layout.
 bool gemv_kimage_format(int ttype) { return kimage_format(ttype); }
+bool gemv_kimage_own(int ttype) { return kimage_own(ttype); }
+long gemv_image_row_bytes(int ttype, int cols, long row_bytes) { return kimage_row_bytes(ttype, cols, row_bytes); }
 
 // GGUF rows -> K-quant image rows; one thread per (row, unit).  The GGUF
 // bytes are read 4-byte (Q4_K) or 2-byte (Q6_K: 210-byte super-blocks)
@@ -396,13 +398,30 @@ __global__ __launch_bounds__(256) void k_kimg_prepare(const uint8_t* __restrict_
   }
 }
 
+// Q2_K, Q3_K and Q5_K rows -> their GEMV image (ImgUnit); one thread per unit
+template <int TT>
+__global__ __launch_bounds__(256) void k_own_prepare(const uint8_t* __restrict__ W, uint8_t* __restrict__ img,
+                                                      long units, int U, long row_bytes, long img_row_bytes) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= units) return;
+  const long row = i / U;
+  ImgUnit<TT>::prepare(W + row * row_bytes, img + row * img_row_bytes, (int)(i - row * U), U);
+}
+
 hipError_t launch_kimage_prepare(int ttype, const void* w, long row_bytes, int rows, int cols, void* img,
                                  hipStream_t s) {
-  if (!kimage_format(ttype) || cols <= 0 || cols % 256) return hipErrorInvalidValue;
+  if (!(kimage_format(ttype) || kimage_own(ttype)) || cols <= 0 || cols % 256) return hipErrorInvalidValue;
   const int U = cols / 64;
   const long units = (long)rows * U;
   if (units <= 0) return hipSuccess;
   const dim3 grid((unsigned)((units + 255) / 256));
+  if (kimage_own(ttype)) {
+    const long irb = kimage_row_bytes(ttype, cols, row_bytes);
+    auto* const f = ttype == TT_Q2_K ? k_own_prepare<TT_Q2_K>
+                    : ttype == TT_Q3_K ? k_own_prepare<TT_Q3_K> : k_own_prepare<TT_Q5_K>;
+    hipLaunchKernelGGL(f, grid, dim3(256), 0, s, (const uint8_t*)w, (uint8_t*)img, units, U, row_bytes, irb);
+    return hipGetLastError();
+  }
   if (ttype == TT_Q4_K)
     hipLaunchKernelGGL(k_kimg_prepare<TT_Q4_K>, grid, dim3(256), 0, s, (const uint8_t*)w, (uint8_t*)img, units, U,
                        row_bytes);

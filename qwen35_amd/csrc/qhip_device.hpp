@@ -868,15 +868,15 @@ struct KImg<TT_Q6_K> {
   }
 };
 
-// a unit's weights from the GGUF row or, IMG, from the K-quant image row
-template <int TT, bool IMG>
-__device__ __forceinline__ typename Unit<TT>::W load_unit(const uint8_t* row, int u, int U) {
-  if constexpr (IMG) return KImg<TT>::load(row, u, U);
-  else return Unit<TT>::load_w(row, u);
-}
-
+// Formats with a K-quant image behind the C ABI, and those whose image only the
+// Exec mirror uses (its rows are not the GGUF rows' bytes).
 constexpr bool kimage_format(int tt) { return tt == TT_Q4_K || tt == TT_Q6_K; }
-
+constexpr bool kimage_own(int tt) { return tt == TT_Q2_K || tt == TT_Q3_K || tt == TT_Q5_K; }
+// bytes of an image row; ImgUnit<tt>'s are padded to whole 16-byte loads
+__host__ __device__ constexpr long kimage_row_bytes(int tt, int cols, long gguf_row_bytes) {
+  return kimage_own(tt) ? ((tt == TT_Q2_K ? 84L : tt == TT_Q3_K ? 114L : 180L) * (cols / 256) + 15) & ~15L
+                        : gguf_row_bytes;
+}
 
 // ---- the further K-quant family (Q8_K activations, 64-value quarter units) ----
 // Every unit below covers values 64c..64c+63 of super-block u>>2 (c = u&3) in
@@ -1053,6 +1053,187 @@ struct Unit<TT_Q2_K> {
     return dall * (float)s[0] - dmin * (float)s[1];
   }
 };
+
+// Units of a GEMV image that holds each unit's own bits.  In the GGUF rows a
+// Q3_K or Q5_K unit re-reads the 32 bytes of high bits that its super-block's
+// four units share, a Q2_K or Q3_K unit twice the low bits it needs, and all of
+// them the packed scales: 78, 80 and 40 bytes loaded for 27.5, 44 and 21, and
+// the bits sorted again in every pass.  An image row is a sequence of planes,
+// one per part, each with the row's U units (or U / 4 super-blocks) in order, so
+// that a team's loads are contiguous.  The integers and the float expression are
+// Unit<TT>'s.
+template <int TT>
+struct ImgUnit;
+
+// 16 bytes of low bits at 16 u (dword i, byte b, bits 2k: value 16 k + 4 i + b),
+// 8 of high bits at 16 U + 8 u (dword i / 2, byte b, bit 4 (i & 1) + k), the
+// int8 scales (sc - 32) at 24 U + 4 u, the super-block's f16 d at 28 U + 2 sb
+template <>
+struct ImgUnit<TT_Q3_K> {
+  struct W { uint32_t lo[4], hi[2], sc, d; };
+  using A = ActQ8K;
+  static __device__ __forceinline__ W load(const uint8_t* row, int u, int U) {
+    W w;
+    const u32x4 l = ld128(row + 16L * u);
+    const uint2 h = *(const uint2*)(row + 16L * U + 8 * u);
+    w.lo[0] = l.x; w.lo[1] = l.y; w.lo[2] = l.z; w.lo[3] = l.w;
+    w.hi[0] = h.x; w.hi[1] = h.y;
+    w.sc = ld32(row + 24L * U + 4 * u);
+    w.d = *(const uint16_t*)(row + 28L * U + 2 * (u >> 2));
+    return w;
+  }
+  static __device__ __forceinline__ void prepare(const uint8_t* src, uint8_t* row, int u, int U) {
+    const uint8_t* blk = src + 110L * (u >> 2);
+    const int c = u & 3, h = c >> 1;
+    uint32_t lo[4] = {0, 0, 0, 0}, hi[2] = {0, 0}, sc = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int g = 2 * (c & 1) + (k >> 1), grp = 4 * c + k;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int at = 16 * (k & 1) + 4 * i;
+        lo[i] |= ((*(const u32_a2*)(blk + 32 + 32 * h + at) >> (2 * g)) & 0x03030303u) << (2 * k);
+        hi[i >> 1] |= ((*(const u32_a2*)(blk + at) >> (4 * h + g)) & 0x01010101u) << (4 * (i & 1) + k);
+      }
+      const uint32_t s6 = ((blk[96 + (grp & 7)] >> (4 * (grp >> 3))) & 15u) |
+                          (((blk[104 + (grp & 3)] >> (2 * (grp >> 2))) & 3u) << 4);
+      sc |= ((s6 - 32u) & 0xFFu) << (8 * k);
+    }
+    *(u32x4*)(row + 16L * u) = u32x4{lo[0], lo[1], lo[2], lo[3]};
+    *(uint2*)(row + 16L * U + 8 * u) = make_uint2(hi[0], hi[1]);
+    *(uint32_t*)(row + 24L * U + 4 * u) = sc;
+    if (c == 0) *(uint16_t*)(row + 28L * U + 2 * (u >> 2)) = *(const uint16_t*)(blk + 108);
+  }
+  static __device__ __forceinline__ A load_a(const uint8_t* act, int u) { return Unit<TT_Q4_K>::load_a(act, u); }
+  static __device__ __forceinline__ float dot(const W& w, const A& a) {
+    int isum = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      int sk = -4 * a.bs[k];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int bit = 4 * (i & 1) + k;
+        const uint32_t h = bit >= 2 ? w.hi[i >> 1] >> (bit - 2) : w.hi[i >> 1] << (2 - bit);
+        sk = dot4(((w.lo[i] >> (2 * k)) & 0x03030303u) | (h & 0x04040404u), a.y[4 * k + i], sk);
+      }
+      isum += sext8(w.sc >> (8 * k)) * sk;
+    }
+    return (h2f(w.d) * a.d) * (float)isum;
+  }
+};
+
+// the GGUF nibbles (qs 32 c..) as two planes of 16 bytes at 16 u and 16 (U + u),
+// 8 bytes of high bits at 32 U + 8 u (dword s, byte b, bit i: sub-block s, value
+// 4 i + b), the scales and mins (sc0, sc1, m0, m1) at 40 U + 4 u, the
+// super-block's d and dmin at 44 U + 4 sb
+template <>
+struct ImgUnit<TT_Q5_K> {
+  struct W { uint32_t q[8], hi[2], sm, dd; };
+  using A = ActQ8K;
+  static __device__ __forceinline__ W load(const uint8_t* row, int u, int U) {
+    W w;
+    const u32x4 a = ld128(row + 16L * u), b = ld128(row + 16L * (U + u));
+    const uint2 h = *(const uint2*)(row + 32L * U + 8 * u);
+    w.q[0] = a.x; w.q[1] = a.y; w.q[2] = a.z; w.q[3] = a.w;
+    w.q[4] = b.x; w.q[5] = b.y; w.q[6] = b.z; w.q[7] = b.w;
+    w.hi[0] = h.x; w.hi[1] = h.y;
+    w.sm = ld32(row + 40L * U + 4 * u);
+    w.dd = ld32(row + 44L * U + 4 * (u >> 2));
+    return w;
+  }
+  static __device__ __forceinline__ void prepare(const uint8_t* src, uint8_t* row, int u, int U) {
+    const Unit<TT_Q5_K>::W w = Unit<TT_Q5_K>::load_w(src, u);
+    const uint32_t S0 = w.hdr[1], S1 = w.hdr[2], S2 = w.hdr[3];
+    const bool upper = w.c >= 2;
+    const uint32_t scw = upper ? ((S2 & 0x0F0F0F0Fu) | ((S0 >> 2) & 0x30303030u)) : (S0 & 0x3F3F3F3Fu);
+    const uint32_t mnw = upper ? (((S2 >> 4) & 0x0F0F0F0Fu) | ((S1 >> 2) & 0x30303030u)) : (S1 & 0x3F3F3F3Fu);
+    const uint32_t sh = 16u * (uint32_t)(w.c & 1);
+    uint32_t h0 = 0, h1 = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      h0 |= ((w.qh[i] >> (2 * w.c)) & 0x01010101u) << i;
+      h1 |= ((w.qh[i] >> (2 * w.c + 1)) & 0x01010101u) << i;
+    }
+    *(u32x4*)(row + 16L * u) = u32x4{w.q[0], w.q[1], w.q[2], w.q[3]};
+    *(u32x4*)(row + 16L * (U + u)) = u32x4{w.q[4], w.q[5], w.q[6], w.q[7]};
+    *(uint2*)(row + 32L * U + 8 * u) = make_uint2(h0, h1);
+    *(uint32_t*)(row + 40L * U + 4 * u) = ((scw >> sh) & 0xFFFFu) | (((mnw >> sh) & 0xFFFFu) << 16);
+    if (w.c == 0) *(uint32_t*)(row + 44L * U + 4 * (u >> 2)) = w.hdr[0];
+  }
+  static __device__ __forceinline__ A load_a(const uint8_t* act, int u) { return Unit<TT_Q4_K>::load_a(act, u); }
+  static __device__ __forceinline__ float dot(const W& w, const A& a) {
+    int lo = 0, hi = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t h0 = i <= 4 ? w.hi[0] << (4 - i) : w.hi[0] >> (i - 4);
+      const uint32_t h1 = i <= 4 ? w.hi[1] << (4 - i) : w.hi[1] >> (i - 4);
+      lo = dot4((w.q[i] & 0x0F0F0F0Fu) | (h0 & 0x10101010u), a.y[i], lo);
+      hi = dot4(((w.q[i] >> 4) & 0x0F0F0F0Fu) | (h1 & 0x10101010u), a.y[8 + i], hi);
+    }
+    const int s = (int)(w.sm & 0xFFu) * lo + (int)((w.sm >> 8) & 0xFFu) * hi;
+    const int m = (int)((w.sm >> 16) & 0xFFu) * (a.bs[0] + a.bs[1]) + (int)(w.sm >> 24) * (a.bs[2] + a.bs[3]);
+    const float d = a.d * h2f(w.dd);
+    const float dmin = a.d * h2f(w.dd >> 16);
+    return d * (float)s - dmin * (float)m;
+  }
+};
+
+// 16 bytes of values at 16 u (as Q3_K's low bits), the GGUF scale bytes 4 c.. at
+// 16 U + 4 u, the super-block's d and dmin at 20 U + 4 sb
+template <>
+struct ImgUnit<TT_Q2_K> {
+  struct W { uint32_t q[4], sc, dd; };
+  using A = ActQ8K;
+  static __device__ __forceinline__ W load(const uint8_t* row, int u, int U) {
+    W w;
+    const u32x4 l = ld128(row + 16L * u);
+    w.q[0] = l.x; w.q[1] = l.y; w.q[2] = l.z; w.q[3] = l.w;
+    w.sc = ld32(row + 16L * U + 4 * u);
+    w.dd = ld32(row + 20L * U + 4 * (u >> 2));
+    return w;
+  }
+  static __device__ __forceinline__ void prepare(const uint8_t* src, uint8_t* row, int u, int U) {
+    const Unit<TT_Q2_K>::W w = Unit<TT_Q2_K>::load_w(src, u);
+    uint32_t q[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        q[i] |= ((w.q[4 * (k & 1) + i] >> (2 * (2 * (w.c & 1) + (k >> 1)))) & 0x03030303u) << (2 * k);
+    *(u32x4*)(row + 16L * u) = u32x4{q[0], q[1], q[2], q[3]};
+    *(uint32_t*)(row + 16L * U + 4 * u) = w.sc;
+    if (w.c == 0) *(uint32_t*)(row + 20L * U + 4 * (u >> 2)) = w.dd;
+  }
+  static __device__ __forceinline__ A load_a(const uint8_t* act, int u) { return Unit<TT_Q4_K>::load_a(act, u); }
+  static __device__ __forceinline__ float dot(const W& w, const A& a) {
+    int isum = 0, summs = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      int sk = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sk = dot4((w.q[i] >> (2 * k)) & 0x03030303u, a.y[4 * k + i], sk);
+      const uint32_t b = (w.sc >> (8 * k)) & 0xFFu;
+      isum += (int)(b & 15u) * sk;
+      summs += (int)(b >> 4) * a.bs[k];
+    }
+    const float dall = a.d * h2f(w.dd);
+    const float dmin = a.d * h2f(w.dd >> 16);
+    return dall * (float)isum - dmin * (float)summs;
+  }
+};
+
+// a row's unit type, from the GGUF row or, IMG, from the K-quant image row
+template <int TT, bool IMG, bool OWN = IMG && kimage_own(TT)>
+struct UnitOf { using type = Unit<TT>; };
+template <int TT, bool IMG>
+struct UnitOf<TT, IMG, true> { using type = ImgUnit<TT>; };
+
+template <int TT, bool IMG>
+__device__ __forceinline__ typename UnitOf<TT, IMG>::type::W load_unit(const uint8_t* row, int u, int U) {
+  if constexpr (IMG && kimage_own(TT)) return ImgUnit<TT>::load(row, u, U);
+  else if constexpr (IMG) return KImg<TT>::load(row, u, U);
+  else return Unit<TT>::load_w(row, u);
+}
 
 template <>
 struct Unit<TT_IQ4_XS> {

@@ -14,7 +14,7 @@ struct GemvArgs {
   int rows, cols, tokens;
   long row_bytes;    // bytes of one weight row
   long act_bytes;    // bytes of one quantized activation row
-  bool kimg = false;  // w is a Q4_K / Q6_K GEMV image (one token)
+  bool kimg = false;  // w is a K-quant GEMV image (one token)
 };
 
 hipError_t launch_quantize_q8_0(const float* x, void* out, long nblocks, int tokens, long x_stride,
@@ -128,6 +128,10 @@ bool gemv_image_preferred(const GemvArgs& g);
 // per row, read by launch_gemv / launch_gemv_fused / launch_gemv_splitk when
 // g.kimg, with the reference Q8_K activation
 bool gemv_kimage_format(int ttype);
+// a format whose K-quant image only the Exec mirror uses, and the bytes of an
+// image row (the GGUF row's, but for those formats)
+bool gemv_kimage_own(int ttype);
+long gemv_image_row_bytes(int ttype, int cols, long row_bytes);
 hipError_t launch_kimage_prepare(int ttype, const void* w, long row_bytes, int rows, int cols, void* img,
                                  hipStream_t s);
 // whether the Exec mirror's batch-1 matvec reads a K-quant weight's image
