@@ -402,22 +402,25 @@ int qhip_backend_wrap_linear(qhip_backend *be, int ttype, int rows, int cols, co
 void qhip_backend_free_linear(qhip_backend *be, qhip_linear *w);
 /* Build what this weight's products use beyond its GGUF bytes now, at load
  * time, instead of inside the first matvec: the GEMV image of an IQ4_NL /
- * Q4_0 / Q8_0 weight large enough for the decode matvec to read it, or of a
- * Q6_K weight whose decode matvec quantizes separately (widths above 4096, or
- * more than 32768 rows)
- * (qhip_launch_gemv_prepare, the GGUF bytes once more; built in load order,
- * so adjacent weights get adjacent images and matvecPair stays one launch),
- * the fragment image of a Q6_K or Q4_K weight with rows * cols >= 2^23
+ * Q4_0 / Q8_0 weight large enough for the decode matvec to read it (past 2^23
+ * weights, 2^25 where the one-launch quantize + GEMV takes the shape), or of a
+ * Q6_K, Q5_K or Q2_K weight whose decode matvec quantizes separately (widths
+ * above 4096, or more than 32768 rows) or a Q3_K weight of more than 2^23
+ * values (the GGUF bytes once more, Q3_K 1.04x and Q5_K 1.02x; built in
+ * load order, so adjacent weights get adjacent images and matvecPair stays one
+ * launch), the fragment image of a Q6_K or Q4_K weight with rows * cols >= 2^23
  * (qhip_launch_wd_prepare, the GGUF bytes once more; matvec_batch_k reads it
  * from 2 tokens, Q6_K up to 64) or of a Q8_0 weight with cols <= 1024 (from
- * 6 tokens) and the MMQ image of a Q6_K weight
- * (qhip_launch_mmq_prepare, 2.5x the GGUF bytes; from 65 tokens).
+ * 6 tokens) and the plane image of the other super-block formats' and Q6_K's
+ * prompts (Q6_K, IQ4_XS and the IQ3 formats 2.02 bytes a weight, Q5_K 2.16,
+ * Q3_K 1.02, Q2_K 1.16; read from 65 tokens, Q3_K from 25, IQ4_XS and the
+ * IQ3 formats from 129).
  * 0 = built or nothing to build; QHIP_DECLINE = not all built (images off, or
  * past the memory budget): the products then read the GGUF bytes.
  * No reference counterpart (its CUDA kernels decode the GGUF blocks in every
  * launch). */
 int qhip_backend_prepare_linear(qhip_backend *be, const qhip_linear *w);
-/* MMQ images (the fragment images and the Q6_K MMQ image) on (default) or
+/* MMQ images (the fragment and plane images) on (default) or
  * off; off, matvec_batch_k never builds or reads one. */
 int qhip_backend_set_mmq_images(qhip_backend *be, int on);
 /* GEMV images on (default) or off; off, matvec never builds or reads one. */

@@ -251,9 +251,9 @@ static hipError_t ensure_skwork(qhip_backend* be, size_t bytes) {
 
 static constexpr int kImgMmq = 0, kImgFrag = 1;
 
-// An MMQ image of a Q6_K weight: looked up, or built now when images are on,
-// the budget allows it and the stream is not being captured (building
-// allocates).  nullptr = run the MMQ on the GGUF bytes instead.
+// An MMQ image of a weight: looked up, or built now when images are on, the
+// budget and the card's memory allow it and the stream is not being captured
+// (building allocates).  nullptr = run the MMQ on the GGUF bytes instead.
 static void* image_for(qhip_backend* be, const void* wdev, int ttype, int rows, int cols, int kind,
                        hipError_t* err) {
   *err = hipSuccess;
@@ -266,7 +266,8 @@ static void* image_for(qhip_backend* be, const void* wdev, int ttype, int rows, 
   void* img = nullptr;
   hipError_t e = hipMalloc(&img, (size_t)n);
   if (e != hipSuccess) {
-    *err = e;
+    if (e == hipErrorOutOfMemory) (void)hipGetLastError();  // the product runs without the image
+    else *err = e;
     return nullptr;
   }
   const int rc = kind == kImgFrag
@@ -288,6 +289,12 @@ static void* image_for(qhip_backend* be, const void* wdev, int ttype, int rows, 
 static size_t act_bytes_for(int cols, int k) {
   const size_t c = (size_t)((cols + 255) / 256) * 256;
   return c / 256 * 292 * (size_t)k + 256;
+}
+
+// Whether the activation scratch holds `bytes`, or may grow to it now.
+static bool act_room(const qhip_backend* be, size_t bytes) {
+  return be->act_cap >= bytes ||
+         (!capturing(be->stream) && !over_budget(be, be->graph_seen ? bytes : bytes - be->act_cap));
 }
 
 // memo family of the split activation the GEMV image reads: kFamSplit plus
@@ -439,8 +446,10 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
   }
   {
     // a prompt: the MMQ from the weight's plane image, on the activation image
+    // (whole groups of 32 tokens: where the scratch has room for the tokens'
+    // Q8_K rows only, the product runs on those)
     const GemvArgs gp{ttype, wdev, x, out, rows, cols, k, row_bytes, qhip_act_row_bytes(ttype, cols)};
-    if (planes_preferred(gp)) {
+    if (planes_preferred(gp) && act_room(be, (size_t)planes_act_bytes(cols, k))) {
       hipError_t e;
       const void* img = image_for(be, wdev, ttype, rows, cols, kImgMmq, &e);
       if (e != hipSuccess) return report("MMQ image", e);
@@ -776,7 +785,9 @@ int qhip_backend_alloc_scratch(qhip_backend* be, int max_cols) {
 
 int qhip_backend_alloc_scratch_k(qhip_backend* be, int max_cols, int k) {
   if (!be || max_cols <= 0 || k <= 0) return (int)hipErrorInvalidValue;
-  return report("scratch", ensure_act(be, act_bytes_for(max_cols, k)));
+  // the activation image of a prompt is of whole 32-token groups
+  const size_t rows = act_bytes_for(max_cols, k), groups = act_bytes_for(max_cols, (k + 31) / 32 * 32);
+  return report("scratch", ensure_act(be, k > 16 && act_room(be, groups) ? groups : rows));
 }
 
 void qhip_backend_free_scratch(qhip_backend* be) {

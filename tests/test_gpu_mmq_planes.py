@@ -140,7 +140,8 @@ def test_planes_captured_and_memo(gpu, oracle, backend):
     family does not meet it."""
     tt, rows, cols, tokens = po.TT_Q5_K, 300, 1024, 150
     w = synth.make_weight(tt, rows, cols, seed=48)
-    lin = backend.wrap_linear(tt, rows, cols, to_dev(w, gpu))
+    wd = to_dev(w, gpu)
+    lin = backend.wrap_linear(tt, rows, cols, wd)
     assert backend.prepare_linear(lin) == 0
     xs = [synth.make_act(cols, tokens, seed=49 + i) for i in range(3)]
     x, out = to_dev(xs[0], gpu), torch.empty((tokens, rows), device=gpu)
@@ -165,8 +166,40 @@ def test_planes_captured_and_memo(gpu, oracle, backend):
     backend.matvec_batch_k(first, lin, x, tokens)
     backend.matvec_batch_k(second, lin, x, tokens)
     backend.set_mmq_images(False)  # another weight without an image: its GGUF rows, on Q8_K rows
-    backend.matvec_batch_k(few, backend.wrap_linear(tt, rows, cols, to_dev(w, gpu).clone()), x, tokens)
+    other = wd.clone()
+    backend.matvec_batch_k(few, backend.wrap_linear(tt, rows, cols, other), x, tokens)
     backend.set_mmq_images(True)
     assert torch.equal(first, second) and rel_l2(few.cpu().numpy(), first.cpu().numpy()) < 1e-6
     h1, m1 = backend.act_stats()
     assert (h1 - h0, m1 - m0) == (1, 2)
+
+
+@pytest.mark.parametrize("room", [True, False])
+def test_planes_captured_after_reservation(gpu, oracle, backend, room):
+    """alloc_scratch_k and prepare_linear make a prompt capturable without an
+    eager run before it, also at a token count that is no whole group of 32;
+    where the budget holds only the Q8_K rows, the product runs on those."""
+    tt, rows, cols, tokens = po.TT_Q3_K, 300, 1024, 37
+    w = synth.make_weight(tt, rows, cols, seed=51)
+    wd = to_dev(w, gpu)
+    lin = backend.wrap_linear(tt, rows, cols, wd)
+    assert backend.prepare_linear(lin) == 0
+    placed = backend.mem_placed()
+    if not room:
+        backend.set_mem_budget(placed + cols // 256 * 292 * tokens + 256)
+    assert backend.lib.qhip_backend_alloc_scratch_k(backend._h, cols, tokens) == 0
+    assert (backend.mem_placed() - placed >= cols // 256 * 292 * 64) == room
+    x, out = torch.empty((tokens, cols), device=gpu), torch.empty((tokens, rows), device=gpu)
+    side = torch.cuda.Stream()
+    backend.set_stream(side)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        backend.matvec_batch_k(out, lin, x, tokens)
+    for i in range(3):
+        xi = synth.make_act(cols, tokens, seed=52 + i)
+        x.copy_(to_dev(xi, gpu))
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert rel_l2(out.cpu().numpy(), oracle.matvec(tt, w, xi)) < TOL
+    backend.set_stream(torch.cuda.current_stream())
