@@ -405,8 +405,9 @@ void qhip_backend_free_linear(qhip_backend *be, qhip_linear *w);
  * Q4_0 / Q8_0 weight large enough for the decode matvec to read it (past 2^23
  * weights, 2^25 where the one-launch quantize + GEMV takes the shape), or of a
  * Q6_K, Q5_K or Q2_K weight whose decode matvec quantizes separately (widths
- * above 4096, or more than 32768 rows) or a Q3_K weight of more than 2^23
- * values (the GGUF bytes once more, Q3_K 1.04x and Q5_K 1.02x; built in
+ * above 4096, or more than 32768 rows) or a Q3_K weight of width 2560 or more and
+ * more than 2^23 values (Q5_K and Q3_K: none narrower than 2560, Q2_K 4096;
+ * the GGUF bytes once more, Q3_K 1.04x and Q5_K 1.02x; built in
  * load order, so adjacent weights get adjacent images and matvecPair stays one
  * launch), the fragment image of a Q6_K or Q4_K weight with rows * cols >= 2^23
  * (qhip_launch_wd_prepare, the GGUF bytes once more; matvec_batch_k reads it

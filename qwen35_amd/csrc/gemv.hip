@@ -1203,9 +1203,16 @@ bool gemv_splitk_preferred(const GemvArgs& g) {
 // and 18.7 / 18.5) and lose where it is (Q2_K [19456, 2560] 10.5 / 8.9, Q5_K
 // [4096, 4096] 7.2 / 6.7).  Q3_K, whose GGUF unit is the dearest, wins there
 // too ([19456, 2560] 12.2 / 15.9, [4096, 4096] 6.5 / 7.3, [2560, 4096] 5.9 /
-// 6.4), so it takes the image from 2^23 weights.
+// 6.4), so it takes the image from 2^23 weights.  Rows of fewer than 40 units
+// leave most lanes of these images' two-wave teams idle and keep the GGUF rows
+// (Q3_K, both with the quantize: [16384, 1024] 10.3 against 6.7 us, [65536,
+// 1024] 26.1 / 17.2, [32768, 1536] 15.9 / 11.6, [16384, 2048] 10.6 / 9.0; from
+// 2560 [5120, 2560] 7.1 / 10.1, [14336, 4096] 9.8 / 14.1; of more than 32768
+// rows Q5_K [65536, 2560] 30.9 / 32.7, Q3_K 27.4 / 41.6), as does Q2_K below
+// 4096 ([65536, 2560] 22.2 / 18.8, [65536, 4096] 20.1 / 29.2).
 bool gemv_kimage_preferred(const GemvArgs& g) {
   if (g.tokens != 1 || g.cols % 256 || !(g.ttype == TT_Q6_K || kimage_own(g.ttype))) return false;
+  if (kimage_own(g.ttype) && g.cols < (g.ttype == TT_Q2_K ? 4096 : 2560)) return false;
   return !gemv_fused_preferred(g) || (g.ttype == TT_Q3_K && (long)g.rows * g.cols > (1L << 23));
 }
 

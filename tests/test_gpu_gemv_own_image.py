@@ -60,10 +60,11 @@ def test_own_image_gemv(gpu, oracle, backend, tt, rows, cols):
 
 
 def test_q3_image_on_short_rows(gpu, oracle, backend):
-    """Q3_K takes the image at widths where the others quantize in the launch."""
-    for tt, rows, uses in ((po.TT_Q3_K, 3645, True), (po.TT_Q3_K, 3640, False), (po.TT_Q2_K, 3645, False),
-                           (po.TT_Q5_K, 3645, False)):
-        cols = 2304
+    """Q3_K takes the image at widths where the others quantize in the launch,
+    from 2560 (40 units)."""
+    for tt, rows, cols, uses in ((po.TT_Q3_K, 3277, 2560, True), (po.TT_Q3_K, 3276, 2560, False),
+                                 (po.TT_Q3_K, 3645, 2304, False), (po.TT_Q3_K, 32775, 256, False),
+                                 (po.TT_Q2_K, 3277, 2560, False), (po.TT_Q5_K, 3277, 2560, False)):
         w = synth.make_weight(tt, rows, cols, seed=53, tag=rows)
         x = synth.make_act(cols, 1, seed=54, tag=1)
         xd = torch.from_numpy(x).to(gpu)
