@@ -118,10 +118,19 @@ static bool mmq_supported(int ttype) {
 // [9728, 2560] x 64 19.1 vs 18.4); Q6_K up to 64 tokens reads its fragment
 // image.  Q4_K stays on its fragment image, a quarter of the bytes: 512 tokens
 // [17408, 5120] 125 us against 133 from its planes.
+//
+// Q5_K to 128 tokens and Q6_K to 96 on rows below 12288 stay on the fragment
+// image, a third of the bytes, whose few-token launch needs no hand-off (us,
+// fragments / planes: Q5_K x 65 [9728, 2560] 20.3 / 33.5, [5120, 17408] 48.3 /
+// 63.9, x 128 [17408, 5120] 61.7 / 71.7, [5120, 17408] 64.5 / 66.6, x 160 84.5 /
+// 75.6; Q6_K x 96 [9728, 2560] 26.3 / 31.7, [2560, 9728] 26.8 / 34.7, [17408,
+// 5120] 62.7 / 66.8, [5120, 17408] 66.5 / 60.3).
+bool wd_image_preferred(const GemvArgs& g);
 bool planes_preferred(const GemvArgs& g) {
   if (g.tokens > 65535 || planes_image_bytes(g.ttype, g.rows, g.cols) <= 0 || !fast_ok(g)) return false;
   switch (g.ttype) {
-    case TT_Q6_K: case TT_Q5_K: case TT_Q2_K: return g.tokens > 64;
+    case TT_Q6_K: case TT_Q5_K: return g.tokens > 64 && !wd_image_preferred(g);
+    case TT_Q2_K: return g.tokens > 64;
     case TT_Q3_K: return g.tokens > 24;
     case TT_IQ4_XS: case TT_IQ3_XXS: case TT_IQ3_S: return g.tokens > 128;
     default: return false;
@@ -143,6 +152,12 @@ bool planes_preferred(const GemvArgs& g) {
 // the plane image and about 50 from the GGUF-row MMQ), the plane image
 // beyond.
 //
+// Q5_K [9728, 2560] 9.8 / 10.2 / 13.2 / 17.4 us at 2 / 8 / 24 / 64 tokens from the
+// image, quantize and product, against 12.7 / 17.8 / 18.2 / 24.8 from the GGUF
+// rows; [17408, 5120] 18.8 / 20.2 / 27.0 / 38.5 against 24.2 / 36.4 / 37.0 / 52.3;
+// [5120, 17408] 19.6 / 21.9 / 28.9 / 48.0 against 33.4 / 39.0 / 40.0 / 52.6;
+// [2560, 9728] 13.2 / 13.9 / 18.8 / 21.1 against 21.4 / 22.0 / 22.4 / 28.6.
+//
 // Q8_0 (the image MMQ from 6 tokens where K is one 1024-value super-chunk):
 // measured on MI355X, [3584, 1024] GEMV 3.59 / 4.36 / 4.84 / 7.84 / 14.02 us
 // at 4 / 6 / 8 / 16 / 32 tokens against 4.23 / 4.25 / 4.32 / 4.47 / 4.90
@@ -155,7 +170,9 @@ bool wd_image_preferred(const GemvArgs& g) {
   if (g.ttype == TT_Q8_0)
     return g.tokens >= 6 && g.cols <= 1024 && wd_image_bytes(g.ttype, g.rows, g.cols) > 0 && fast_ok(g);
   if (g.tokens < 2 || (long)g.rows * g.cols < (1L << 23) || !fast_ok(g)) return false;
-  if (g.ttype == TT_Q6_K) return g.tokens <= 64 && wd_image_bytes(g.ttype, g.rows, g.cols) > 0;
+  const int most = g.ttype == TT_Q5_K ? 128 : g.ttype == TT_Q6_K ? (g.cols < 12288 ? 96 : 64) : 0x7FFFFFFF;
+  if (g.tokens > most || wd_image_bytes(g.ttype, g.rows, g.cols) <= 0) return false;
+  if (g.ttype == TT_Q6_K || g.ttype == TT_Q5_K) return true;
   return g.ttype == TT_Q4_K && wd_image_bytes(g.ttype, g.rows, g.cols) > 0;
 }
 
@@ -499,11 +516,14 @@ int qhip_launch_mul_mat_image(const void* d_image, const void* d_xq, float* d_ou
   return (int)launch_mmq_image(g, tile_tokens, tile_rows, d_work, d_work ? work_bytes : 0, S(stream));
 }
 
-long qhip_wd_image_bytes(int ttype, int rows, int cols) { return wd_image_bytes(ttype, rows, cols); }
+// the fragment image of Q5_K is the Exec mirror's own
+long qhip_wd_image_bytes(int ttype, int rows, int cols) {
+  return ttype == TT_Q5_K ? -1 : wd_image_bytes(ttype, rows, cols);
+}
 
 int qhip_launch_wd_prepare(int ttype, const void* d_w, int rows, int cols, void* d_image, void* stream) {
   const long rb = weight_row_bytes(ttype, cols);
-  if (rb < 0 || wd_image_bytes(ttype, rows, cols) < 0) return (int)hipErrorInvalidValue;
+  if (rb < 0 || qhip_wd_image_bytes(ttype, rows, cols) < 0) return (int)hipErrorInvalidValue;
   if (rows == 0) return 0;
   if (!d_w || !d_image || ((uintptr_t)d_image & 15u)) return (int)hipErrorInvalidValue;
   return (int)launch_wd_prepare(ttype, d_w, rb, rows, cols, d_image, S(stream));
@@ -514,7 +534,7 @@ int qhip_launch_mul_mat_wd_image(const void* d_image, const void* d_xq, float* d
   GemvArgs g;
   hipError_t e = make_args(d_image, d_xq, d_out, rows, cols, tokens, ttype, g);
   if (e != hipSuccess) return (int)e;
-  if (wd_image_bytes(ttype, rows, cols) < 0 || (ttype == TT_Q6_K && tokens > 64)) return (int)hipErrorInvalidValue;
+  if (qhip_wd_image_bytes(ttype, rows, cols) < 0 || (ttype == TT_Q6_K && tokens > 64)) return (int)hipErrorInvalidValue;
   if (((uintptr_t)d_image & 15u) || !aligned4(d_xq)) return (int)hipErrorInvalidValue;
   if (work_bytes < 0 || (d_work && ((uintptr_t)d_work & 15u))) return (int)hipErrorInvalidValue;
   if (rows == 0 || tokens == 0) return 0;

@@ -261,7 +261,7 @@ static void* image_for(qhip_backend* be, const void* wdev, int ttype, int rows, 
   auto it = be->images.find(key);
   if (it != be->images.end()) return it->second.p;
   if (!be->images_on || capturing(be->stream)) return nullptr;
-  const long n = kind == kImgFrag ? qhip_wd_image_bytes(ttype, rows, cols) : planes_image_bytes(ttype, rows, cols);
+  const long n = kind == kImgFrag ? wd_image_bytes(ttype, rows, cols) : planes_image_bytes(ttype, rows, cols);
   if (n <= 0 || over_budget(be, (size_t)n)) return nullptr;
   void* img = nullptr;
   hipError_t e = hipMalloc(&img, (size_t)n);
@@ -270,10 +270,9 @@ static void* image_for(qhip_backend* be, const void* wdev, int ttype, int rows, 
     else *err = e;
     return nullptr;
   }
-  const int rc = kind == kImgFrag
-                     ? qhip_launch_wd_prepare(ttype, wdev, rows, cols, img, be->stream)
-                     : (int)launch_planes_prepare(ttype, wdev, qhip_weight_row_bytes(ttype, cols), rows, cols, img,
-                                                  be->stream);
+  const long rb = qhip_weight_row_bytes(ttype, cols);
+  const int rc = (int)(kind == kImgFrag ? launch_wd_prepare(ttype, wdev, rb, rows, cols, img, be->stream)
+                                        : launch_planes_prepare(ttype, wdev, rb, rows, cols, img, be->stream));
   if (rc) {
     (void)hipFree(img);
     *err = (hipError_t)rc;
@@ -554,12 +553,13 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
   void* work = be->skwork;
   const long work_bytes = (long)be->skwork_cap;
   if (wd_image_preferred(g)) {
-    // a few tokens of a Q6_K weight: the MMQ from its fragment image
+    // a few tokens of a Q6_K, Q4_K or Q5_K weight: the MMQ from its fragment image
     void* img = image_for(be, wdev, ttype, rows, cols, kImgFrag, &e);
     if (e != hipSuccess) return report("fragment image", e);
     if (img)
-      return report("matvec", (hipError_t)qhip_launch_mul_mat_wd_image(img, be->act, out, rows, cols, k, ttype, work,
-                                                                        work_bytes, be->stream));
+      return report("matvec", launch_mmq_wd_image(GemvArgs{ttype, img, be->act, out, rows, cols, k, row_bytes,
+                                                           qhip_act_row_bytes(ttype, cols)}, work, work_bytes,
+                                                  be->stream, true));
   }
   return report("matvec", dispatch_mul_mat(g, QHIP_PATH_AUTO, work, work_bytes, be->stream));
 }

@@ -1600,7 +1600,20 @@ __global__ __launch_bounds__(256) void k_mmq_wd_q4k(const uint8_t* __restrict__ 
 // sub-block on the raw nibbles, the sub-block scale applied to the integer
 // result on the NE kept elements, the mins through an exact f16 MFMA, then
 // acc[0][0] += dy * (d * isum - dmin * summs).  A macro, as the Q6_K one.
-#define QHIP_Q4K_SUPERBLOCK(wh_, wq_, A, arow)                                                                       \
+// FRAG(c, hi): the MFMA operand of sub-block 2 c + hi (Q4_K: the nibbles; Q5_K:
+// nibble + 16 * its bit 2 c + hi of the high-bit bytes, |isum| < 2^26).
+template <int TT>
+__device__ __forceinline__ i32x4 q45_frag(const u32x4& q, const u32x4& hb, int s) {
+  i32x4 v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t n = (s & 1 ? q[i] >> 4 : q[i]) & 0x0F0F0F0Fu;
+    if constexpr (TT == TT_Q5_K) n |= (s < 4 ? hb[i] << (4 - s) : hb[i] >> (s - 4)) & 0x10101010u;
+    v[i] = (int)n;
+  }
+  return v;
+}
+#define QHIP_Q4K_SUPERBLOCK(wh_, FRAG, A, arow)                                                                      \
   do {                                                                                                               \
     const i32x16 zero_ = {};                                                                                         \
     const f32x16 fz_ = {};                                                                                           \
@@ -1611,11 +1624,9 @@ __global__ __launch_bounds__(256) void k_mmq_wd_q4k(const uint8_t* __restrict__ 
     int isum_[NE];                                                                                                   \
     _Pragma("unroll") for (int e_ = 0; e_ < NE; ++e_) isum_[e_] = 0;                                                 \
     _Pragma("unroll") for (int c_ = 0; c_ < 4; ++c_) {                                                               \
-      const uint32_t q0_ = (wq_)[c_].x, q1_ = (wq_)[c_].y, q2_ = (wq_)[c_].z, q3_ = (wq_)[c_].w;                     \
       _Pragma("unroll") for (int hi_ = 0; hi_ < 2; ++hi_) {                                                          \
         const int s_ = 2 * c_ + hi_;                                                                                 \
-        const i32x4 bq_ = {(int)((hi_ ? q0_ >> 4 : q0_) & 0x0F0F0F0Fu), (int)((hi_ ? q1_ >> 4 : q1_) & 0x0F0F0F0Fu), \
-                          (int)((hi_ ? q2_ >> 4 : q2_) & 0x0F0F0F0Fu), (int)((hi_ ? q3_ >> 4 : q3_) & 0x0F0F0F0Fu)}; \
+        const i32x4 bq_ = FRAG(c_, hi_);                                                                             \
         const int sc_ = (int)(((s_ < 4 ? sc_lo_ : sc_hi_) >> (8 * (s_ & 3))) & 63u);                                 \
         const i32x4 af_ = *(const i32x4*)((A) + (arow) * kWdRow + 32 * s_ + 16 * lh);                                \
         const i32x16 S_ = __builtin_amdgcn_mfma_i32_32x32x32_i8(af_, bq_, zero_, 0, 0, 0);                           \
@@ -1710,7 +1721,8 @@ __global__ __launch_bounds__(256) void k_mmq_wds_q4k(const uint8_t* __restrict__
       issue_act(sb + 1, nxt);
       issue_w(sb + 1, nh, nq);
     }
-    QHIP_Q4K_SUPERBLOCK(wh, wq, A, li);
+    auto frag = [&](int c, int hi) { return q45_frag<TT_Q4_K>(wq[c], wh, 2 * c + hi); };
+    QHIP_Q4K_SUPERBLOCK(wh, frag, A, li);
     __builtin_amdgcn_s_waitcnt(0);  // chunk sb+1: DMA and weight registers
     __syncthreads();
     if (sb + 1 < sb1) {
@@ -1750,6 +1762,10 @@ __global__ __launch_bounds__(256) void k_mmq_wds_q4k(const uint8_t* __restrict__
 //   [6144, 6656)  row i's 16 int8 scales at 6144 + 16 i
 //   [6656, 6720)  row i's f16 d at 6656 + 2 i
 constexpr int kWdiTile = 6720;
+// Q5_K: the Q4_K tile, then each lane's 16 high-bit bytes (values 16 (L / 32)
+// ..+15 of every sub-block s in bit s)
+constexpr int kWdiTile5 = kWdiTile4 + 1024;
+constexpr int wdi_tile(int tt) { return tt == TT_Q6_K ? kWdiTile : tt == TT_Q5_K ? kWdiTile5 : kWdiTile4; }
 
 template <bool IMG>
 struct Q6Regs;
@@ -2056,10 +2072,12 @@ __global__ __launch_bounds__(256) void k_wd_prepare_q6k(const uint8_t* __restric
   }
 }
 
-// One thread per (tile, lane L) of the Q4_K fragment image: lane L's four
-// 16-byte qs pieces; lanes L < 32 also the row's header.  Rows past the end:
-// zeros.  GGUF Q4_K rows are 144 bytes per super-block: every piece aligned.
-__global__ __launch_bounds__(256) void k_wd_prepare_q4k(const uint8_t* __restrict__ W, uint8_t* __restrict__ IMG,
+// One thread per (tile, lane L) of the Q4_K / Q5_K fragment image: lane L's four
+// 16-byte qs pieces (Q5_K: and its qh piece); lanes L < 32 also the row's
+// header.  Rows past the end: zeros.  GGUF super-blocks are 144 / 176 bytes:
+// every piece aligned.
+template <int TT>
+__global__ __launch_bounds__(256) void k_wd_prepare_q45k(const uint8_t* __restrict__ W, uint8_t* __restrict__ IMG,
                                                          int rows, long row_bytes, int nsb, long nthreads) {
   const long gid = (long)blockIdx.x * 256 + threadIdx.x;
   if (gid >= nthreads) return;
@@ -2068,13 +2086,14 @@ __global__ __launch_bounds__(256) void k_wd_prepare_q4k(const uint8_t* __restric
   const long grp = tile / nsb;
   const int sb = (int)(tile - grp * nsb);
   const long row = grp * 32 + i;
-  uint8_t* t = IMG + tile * kWdiTile4;
-  uint4 q[4], h = make_uint4(0u, 0u, 0u, 0u);
+  uint8_t* t = IMG + tile * wdi_tile(TT);
+  uint4 q[4], h = make_uint4(0u, 0u, 0u, 0u), x = h;
   if (row < rows) {
-    const uint8_t* b = W + row * row_bytes + 144L * sb;
+    const uint8_t* b = W + row * row_bytes + (TT == TT_Q5_K ? 176L : 144L) * sb;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) q[c] = *(const uint4*)(b + 16 + 32 * c + 16 * k);
+    for (int c = 0; c < 4; ++c) q[c] = *(const uint4*)(b + (TT == TT_Q5_K ? 48 : 16) + 32 * c + 16 * k);
     h = *(const uint4*)b;
+    if constexpr (TT == TT_Q5_K) x = *(const uint4*)(b + 16 + 16 * k);
   } else {
 #pragma unroll
     for (int c = 0; c < 4; ++c) q[c] = make_uint4(0u, 0u, 0u, 0u);
@@ -2082,6 +2101,7 @@ __global__ __launch_bounds__(256) void k_wd_prepare_q4k(const uint8_t* __restric
 #pragma unroll
   for (int c = 0; c < 4; ++c) *(uint4*)(t + 1024 * c + 16 * L) = q[c];
   if (k == 0) *(uint4*)(t + 4096 + 16 * i) = h;
+  if constexpr (TT == TT_Q5_K) *(uint4*)(t + kWdiTile4 + 16 * L) = x;
 }
 
 // ---- Q8_0 fragment image and its MMQ ----------------------------------------------------
@@ -2694,9 +2714,10 @@ hipError_t launch_mmq_bg_q6k(const GemvArgs& g, void* work, long work_bytes, hip
 }
 
 long wd_image_bytes(int ttype, int rows, int cols) {
-  if ((ttype != TT_Q6_K && ttype != TT_Q4_K && ttype != TT_Q8_0) || rows < 0 || cols <= 0 || cols % 256) return -1;
+  if (ttype != TT_Q6_K && ttype != TT_Q4_K && ttype != TT_Q5_K && ttype != TT_Q8_0) return -1;
+  if (rows < 0 || cols <= 0 || cols % 256) return -1;
   if (ttype == TT_Q8_0) return (long)((rows + 31) / 32) * (cols / 32) * kQ8iBlk;
-  return (long)((rows + 31) / 32) * (cols / 256) * (ttype == TT_Q6_K ? kWdiTile : kWdiTile4);
+  return (long)((rows + 31) / 32) * (cols / 256) * wdi_tile(ttype);
 }
 
 hipError_t launch_wd_prepare(int ttype, const void* w, long row_bytes, int rows, int cols, void* img,
@@ -2716,14 +2737,15 @@ hipError_t launch_wd_prepare(int ttype, const void* w, long row_bytes, int rows,
     hipLaunchKernelGGL(k_wd_prepare_q6k, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (const uint8_t*)w,
                        (uint8_t*)img, rows, row_bytes, nsb, n);
   else
-    hipLaunchKernelGGL(k_wd_prepare_q4k, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (const uint8_t*)w,
-                       (uint8_t*)img, rows, row_bytes, nsb, n);
+    hipLaunchKernelGGL(ttype == TT_Q5_K ? k_wd_prepare_q45k<TT_Q5_K> : k_wd_prepare_q45k<TT_Q4_K>,
+                       dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, (const uint8_t*)w, (uint8_t*)img, rows,
+                       row_bytes, nsb, n);
   return hipGetLastError();
 }
 
 // ---- few tokens, K split inside the workgroup -------------------------------------------
-// T <= 8 NG from a fragment image with no split-K hand-off between
-// workgroups: a workgroup of NW waves owns one group of 32 rows; wave w takes
+// Tiles of 8 NG tokens (blockIdx.y) from a fragment image with no split-K hand-off
+// between workgroups: a workgroup of NW waves owns one group of 32 rows; wave w takes
 // super-blocks [w cpw, (w+1) cpw) of the whole row (its own activation stages
 // in LDS, its weight loads and DMA for CPS super-blocks issued before any of
 // it is used), and the waves' partial sums are added through LDS in wave
@@ -2749,7 +2771,7 @@ __global__ __launch_bounds__(64 * NW) void k_mmq_rk(const uint8_t* __restrict__ 
                                                      int nsb, int cpw) {
   constexpr int TR = 8 * NG, NE = 4 * NG;
   constexpr int STAGE = TR * kWdRow, NPC = TR * kWdPieces, NDW = (CPS * NPC + 63) / 64;
-  constexpr int TILE = TT == TT_Q6_K ? kWdiTile : kWdiTile4;
+  constexpr int TILE = wdi_tile(TT);
   constexpr int LDSB = NW * CPS * STAGE > NW * NE * 256 ? NW * CPS * STAGE : NW * NE * 256;
   __shared__ __attribute__((aligned(16))) uint8_t lds[LDSB];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, li = lane & 31, lh = lane >> 5;
@@ -2757,6 +2779,7 @@ __global__ __launch_bounds__(64 * NW) void k_mmq_rk(const uint8_t* __restrict__ 
   const uint8_t* wbase = W + (long)(grp < ngrp ? grp : ngrp - 1) * nsb * TILE;
   const int sb0 = wv * cpw, sb1 = sb0 + cpw < nsb ? sb0 + cpw : nsb;
   const int arow = li < TR ? li : 0;
+  const int t0 = TR * blockIdx.y;         // this workgroup's tokens
   uint8_t* act = lds + wv * CPS * STAGE;  // this wave's stages
 
   // DMA piece P = 64 i + lane of this wave's run: stage P / (19 TR), token
@@ -2768,7 +2791,7 @@ __global__ __launch_bounds__(64 * NW) void k_mmq_rk(const uint8_t* __restrict__ 
     const int P = 64 * i + lane;
     const int sg = P / NPC, p = P - sg * NPC;
     const int tp = p / kWdPieces, j = p - tp * kWdPieces;
-    const int tok = tp < tokens ? tp : tokens - 1;
+    const int tok = t0 + tp < tokens ? t0 + tp : tokens - 1;
     gst[i] = P < CPS * NPC ? sg : CPS;
     goff[i] = (long)tok * act_bytes + (j < 16 ? 4 + 16 * j : j == 16 ? 260 : j == 17 ? 276 : 0);
   }
@@ -2805,12 +2828,13 @@ __global__ __launch_bounds__(64 * NW) void k_mmq_rk(const uint8_t* __restrict__ 
         }
       }
     } else {
-      u32x4 wh[CPS], wq[CPS][4];
+      u32x4 wh[CPS], wq[CPS][4], wx[CPS] = {};
 #pragma unroll
       for (int s = 0; s < CPS; ++s) {
         if (s < n) {
           const uint8_t* b = wbase + (long)TILE * (base + s);
           wh[s] = *(const u32x4*)(b + 4096 + 16 * li);
+          if constexpr (TT == TT_Q5_K) wx[s] = *(const u32x4*)(b + kWdiTile4 + 16 * lane);
 #pragma unroll
           for (int c = 0; c < 4; ++c) wq[s][c] = *(const u32x4*)(b + 1024 * c + 16 * lane);
         }
@@ -2825,7 +2849,8 @@ __global__ __launch_bounds__(64 * NW) void k_mmq_rk(const uint8_t* __restrict__ 
       for (int s = 0; s < CPS; ++s) {
         if (s < n) {
           const uint8_t* As = act + s * STAGE;
-          QHIP_Q4K_SUPERBLOCK(wh[s], wq[s], As, arow);
+          auto frag = [&](int c, int hi) { return q45_frag<TT>(wq[s][c], wx[s], 2 * c + hi); };
+          QHIP_Q4K_SUPERBLOCK(wh[s], frag, As, arow);
         }
       }
     }
@@ -2843,7 +2868,7 @@ __global__ __launch_bounds__(64 * NW) void k_mmq_rk(const uint8_t* __restrict__ 
       float v = red[e * 64 + lane];
 #pragma unroll
       for (int w = 1; w < NW; ++w) v += red[(w * NE + e) * 64 + lane];
-      const int tok = 8 * (e >> 2) + 4 * lh + (e & 3);
+      const int tok = t0 + 8 * (e >> 2) + 4 * lh + (e & 3);
       if (row < rows && tok < tokens) Y[(long)tok * rows + row] = v;
     }
   }
@@ -3015,44 +3040,88 @@ static hipError_t launch_mmq_wds_q6k(const GemvArgs& g, int ksplit, void* work, 
   return hipGetLastError();
 }
 
-// From the fragment image: Q6_K 1..32 tokens, Q4_K any count; work as for
-// launch_mmq (the same slices as the GGUF-row launch, so mmq_work_bytes
-// covers it).
 template <int TT, int NW>
-static hipError_t launch_mmq_rk(const GemvArgs& g, hipStream_t s) {
+static hipError_t launch_mmq_rk_nw(const GemvArgs& g, hipStream_t s) {
   const int nsb = g.cols / 256, ngrp = (g.rows + 31) / 32;
   const int cpw = (nsb + NW - 1) / NW;
-  const int ng = (g.tokens + 7) / 8;
-#define QHIP_RK(N)                                                                                               \
-  if (ng == N)                                                                                                   \
-    hipLaunchKernelGGL((k_mmq_rk<TT, N, NW, 1>), dim3((unsigned)ngrp), dim3(64 * NW), 0, s, (const uint8_t*)g.w, \
-                       (const uint8_t*)g.xq, g.out, g.rows, g.tokens, g.act_bytes, nsb, cpw);
-  QHIP_RK(1) QHIP_RK(2) QHIP_RK(3)
+  const int ntt = (g.tokens + 31) / 32, ng = ntt > 1 ? 4 : (g.tokens + 7) / 8;
+#define QHIP_RK(N)                                                                                                  \
+  if (ng == N)                                                                                                      \
+    hipLaunchKernelGGL((k_mmq_rk<TT, N, NW, 1>), dim3((unsigned)ngrp, (unsigned)ntt), dim3(64 * NW), 0, s,          \
+                       (const uint8_t*)g.w, (const uint8_t*)g.xq, g.out, g.rows, g.tokens, g.act_bytes, nsb, cpw);
+  QHIP_RK(1) QHIP_RK(2) QHIP_RK(3) QHIP_RK(4)
 #undef QHIP_RK
   return hipGetLastError();
 }
 
+// Waves of a workgroup: with at most one workgroup per CU the waves of a group
+// of rows are all the CU has, so eight, and twelve on long rows; past that four
+// (eight up to 16 tokens within two workgroups per CU), as the stages of more
+// waves keep workgroups off the CU.  Weights from HBM, quantize and product, us
+// with 4 / 8 / 12 waves: Q5_K [4096, 4096] x 64 16.0 / 12.7 / 13.1, [5120, 17408]
+// x 8 31.8 / 22.5 / 20.4, [9728, 2560] x 8 10.8 / 10.2 / 11.5 and x 64 17.5 /
+// 23.7 / 24.7; Q4_K [2560, 9728] x 8 18.5 / 12.7 / 12.3 (all four before);
+// Q6_K [17408, 5120] x 16 26.6 / 27.2 / 30.0 (all twelve before).
+static int rk_waves(const GemvArgs& g) {
+  const int cus0 = qhip_gpu_cu_count(), cus = cus0 > 0 ? cus0 : 256;
+  const long wgs = (long)((g.rows + 31) / 32) * ((g.tokens + 31) / 32);
+  if (wgs <= cus) return g.cols >= 9216 && g.tokens <= 32 ? 12 : 8;
+  return g.tokens <= 16 && wgs <= 2L * cus ? 8 : 4;
+}
+
+// Whether the launch from the fragment image keeps K inside the workgroup: the
+// tokens past 32 run as further 32-token tiles, whose weight reads meet in L2.
+// Against the launches that cut K over workgroups (k_mmq_wd_q4k, k_mmq_wdp_q6k),
+// us as above: Q4_K x 24 [9728, 2560] 12.2 / 13.7 (x 32), [5120, 17408] 26.9 /
+// 23.9, [2560, 9728] 18.0 / 16.2; Q6_K x 32 [9728, 2560] 17.9 / 19.9, [4096,
+// 4096] 14.5 / 18.6, x 64 [17408, 5120] 47.8 / 67.5, [5120, 17408] 64.3 / 48.8,
+// [2560, 9728] 26.3 / 25.4.  Q5_K has no other.  The public image calls (mirror
+// false) keep the GGUF-row launch's K slices, and so its bits, from 17 tokens of
+// Q6_K, and this launch to 24 of Q4_K.
+static bool rk_preferred(const GemvArgs& g, bool mirror) {
+  const int nsb = g.cols / 256;
+  if (g.ttype == TT_Q5_K) return true;
+  if (!mirror) return g.tokens <= (g.ttype == TT_Q4_K ? 24 : 16);
+  if (g.ttype == TT_Q4_K) return g.tokens <= (nsb >= 36 ? 16 : 24);
+  return g.ttype == TT_Q6_K && (g.tokens <= 16 || g.tokens > 64 || nsb <= 20);
+}
+
+template <int TT>
+static hipError_t launch_mmq_rk(const GemvArgs& g, hipStream_t s) {
+  switch (rk_waves(g)) {
+    case 12: return launch_mmq_rk_nw<TT, 12>(g, s);
+    case 8: return launch_mmq_rk_nw<TT, 8>(g, s);
+    default: return launch_mmq_rk_nw<TT, 4>(g, s);
+  }
+}
+
+// the most that either caller's launch splits into
 long wd_image_work_bytes(const GemvArgs& g) {
-  if (g.ttype == TT_Q4_K) return g.tokens <= 24 ? 0 : wd_work_bytes(g, wd_plan(g));
-  if (g.ttype == TT_Q6_K && g.tokens > 16 && g.tokens <= 64) return mmq_split_bytes(g, 32, kWdBR, wds_q6k_slices(g));
+  if (rk_preferred(g, true) && rk_preferred(g, false)) return 0;
+  if (g.ttype == TT_Q4_K) return wd_work_bytes(g, wd_plan(g));
+  if (g.ttype == TT_Q6_K && g.tokens <= 64) return mmq_split_bytes(g, 32, kWdBR, wds_q6k_slices(g));
   return 0;
 }
 
-hipError_t launch_mmq_wd_image(const GemvArgs& g, void* work, long work_bytes, hipStream_t s) {
+// From the fragment image: Q6_K 1..96 tokens, Q5_K 1..128, Q4_K any count; work
+// as for launch_mmq (the same slices as the GGUF-row launch, so mmq_work_bytes
+// covers it).
+hipError_t launch_mmq_wd_image(const GemvArgs& g, void* work, long work_bytes, hipStream_t s, bool mirror) {
   if (g.rows <= 0 || g.tokens <= 0) return hipSuccess;
   if (g.ttype == TT_Q8_0) return launch_mmq_q8i(g, s);
   if (g.ttype == TT_Q4_K) {
-    // up to 24 tokens the K split inside the workgroup; beyond, the 32- and
+    // a few tokens: the K split inside the workgroup; beyond, the 32- and
     // 64-token weights-direct tiles (split over workgroups on small grids)
-    if (g.tokens <= 24) return launch_mmq_rk<TT_Q4_K, 4>(g, s);
+    if (rk_preferred(g, mirror)) return launch_mmq_rk<TT_Q4_K>(g, s);
     WdPlan plan = wd_plan(g);
     if (!work || work_bytes < wd_work_bytes(g, plan)) plan = WdPlan{1, 0};
     return launch_mmq_wd<true>(g, plan, work, s, wd_bt(g));
   }
-  if (g.ttype != TT_Q6_K || g.tokens > 64) return hipErrorInvalidValue;
-  // up to 16 tokens the K split inside the workgroup; 17..32 the split
-  // launch with whole-group prefetch (28.0 against 28.3 us at 24 tokens)
-  if (g.tokens <= 16) return launch_mmq_rk<TT_Q6_K, 12>(g, s);
+  if (g.tokens > 128) return hipErrorInvalidValue;
+  if (g.ttype == TT_Q5_K) return launch_mmq_rk<TT_Q5_K>(g, s);
+  if (g.ttype != TT_Q6_K || g.tokens > 96) return hipErrorInvalidValue;
+  if (rk_preferred(g, mirror)) return launch_mmq_rk<TT_Q6_K>(g, s);
+  // the split launch with whole-group prefetch
   const int ntt = (g.tokens + 31) / 32;
   int ksplit = wds_q6k_slices(g);
   if (!work || work_bytes < mmq_split_bytes(g, 32, kWdBR, ksplit)) ksplit = 1;

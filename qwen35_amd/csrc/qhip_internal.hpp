@@ -103,7 +103,7 @@ hipError_t launch_mmq_bg_q6k(const GemvArgs& g, void* work, long work_bytes, hip
 long wd_image_bytes(int ttype, int rows, int cols);
 hipError_t launch_wd_prepare(int ttype, const void* w, long row_bytes, int rows, int cols, void* img,
                              hipStream_t s);
-hipError_t launch_mmq_wd_image(const GemvArgs& g, void* work, long work_bytes, hipStream_t s);
+hipError_t launch_mmq_wd_image(const GemvArgs& g, void* work, long work_bytes, hipStream_t s, bool mirror = false);
 long mmq_image_work_bytes(const GemvArgs& g);
 // the split-K workspace launch_mmq_wd_image takes (fragment image; 0 = none)
 long wd_image_work_bytes(const GemvArgs& g);
