@@ -10,6 +10,7 @@
 #include "qhip_internal.hpp"
 
 #include <algorithm>
+#include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -94,6 +95,10 @@ struct qhip_backend {
   // then runs the tile MMQ on the GGUF bytes).
   size_t budget = 0;
   size_t placed = 0;  // bytes counted against the budget
+  // The smallest image that the card had no memory for, until prepare_linear
+  // asks again or this backend gives memory back: a matvec without its image
+  // does not try the allocation anew on every call.
+  size_t refused = SIZE_MAX;
   // What `act` holds (backend_cuda.zig:3425-3448 actQValid/actQMark): the
   // source pointer, width, token count and activation family of the last
   // quantization, so a second matvec of the same x skips its quantize.
@@ -155,6 +160,15 @@ static hipError_t budget_error(const qhip_backend* be, const char* what, size_t 
   return hipErrorOutOfMemory;
 }
 
+// hipMalloc, a refusal left to the return value alone: the runtime keeps an
+// error until it is read, and a caller that goes on without the memory would
+// have its next launch's hipGetLastError() return it.
+static hipError_t dev_alloc(void** p, size_t bytes) {
+  const hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+
 static hipError_t arena_alloc(qhip_backend* be, size_t bytes, uint8_t** out) {
   bytes = (bytes + kAlign - 1) / kAlign * kAlign;
   if (over_budget(be, bytes)) return budget_error(be, "weight upload", bytes);
@@ -171,7 +185,7 @@ static hipError_t arena_alloc(qhip_backend* be, size_t bytes, uint8_t** out) {
   size_t sz = bytes > kArenaChunk ? bytes : kArenaChunk;
   if (be->budget && sz > be->budget - be->placed) sz = bytes > be->budget - be->placed ? bytes : be->budget - be->placed;
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, sz);
+  hipError_t e = dev_alloc(&p, sz);
   if (e != hipSuccess) return e;
   be->arena.push_back({(uint8_t*)p, sz, bytes});
   be->placed += bytes;
@@ -217,7 +231,7 @@ static hipError_t ensure_act(qhip_backend* be, size_t bytes) {
   be->act_cap = 0;
   memo_clear(be);
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, bytes);
+  hipError_t e = dev_alloc(&p, bytes);
   if (e != hipSuccess) return e;
   be->act = (uint8_t*)p;
   be->act_cap = bytes;
@@ -234,7 +248,7 @@ static hipError_t ensure_skwork(qhip_backend* be, size_t bytes) {
   be->skwork = nullptr;
   be->skwork_cap = 0;
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, bytes);
+  hipError_t e = dev_alloc(&p, bytes);
   if (e != hipSuccess) return e;
   // the counters start at zero; a fill kernel on the backend's stream orders
   // it before the first split launch
@@ -262,11 +276,11 @@ static void* image_for(qhip_backend* be, const void* wdev, int ttype, int rows, 
   if (it != be->images.end()) return it->second.p;
   if (!be->images_on || capturing(be->stream)) return nullptr;
   const long n = kind == kImgFrag ? wd_image_bytes(ttype, rows, cols) : planes_image_bytes(ttype, rows, cols);
-  if (n <= 0 || over_budget(be, (size_t)n)) return nullptr;
+  if (n <= 0 || over_budget(be, (size_t)n) || (size_t)n >= be->refused) return nullptr;
   void* img = nullptr;
-  hipError_t e = hipMalloc(&img, (size_t)n);
+  hipError_t e = dev_alloc(&img, (size_t)n);
   if (e != hipSuccess) {
-    if (e == hipErrorOutOfMemory) (void)hipGetLastError();  // the product runs without the image
+    if (e == hipErrorOutOfMemory) be->refused = (size_t)n;  // the product runs without the image
     else *err = e;
     return nullptr;
   }
@@ -318,7 +332,8 @@ static hipError_t img_arena_alloc(qhip_backend* be, size_t bytes, uint8_t** out)
   size_t sz = bytes > kArenaChunk ? bytes : kArenaChunk;
   if (be->budget && sz > be->budget - be->placed) sz = bytes;
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, sz);
+  hipError_t e = dev_alloc(&p, sz);
+  if (e == hipErrorOutOfMemory && sz > bytes) e = dev_alloc(&p, sz = bytes);
   if (e != hipSuccess) return e;
   be->img_arena.push_back({(uint8_t*)p, sz, bytes});
   be->placed += bytes;
@@ -364,11 +379,12 @@ static uint8_t* gimage_for(qhip_backend* be, const void* wdev, int ttype, int ro
   if (!be->gemv_images_on || capturing(be->stream)) return nullptr;
   const long irb = gemv_image_row_bytes(ttype, cols, row_bytes);
   const long n = gemv_kimage_own(ttype) ? irb * rows : qhip_gemv_image_bytes(ttype, rows, cols);
-  if (n <= 0 || over_budget(be, (size_t)n)) return nullptr;
+  if (n <= 0 || over_budget(be, (size_t)n) || (size_t)n >= be->refused) return nullptr;
   uint8_t* img = nullptr;
   hipError_t e = img_arena_alloc(be, (size_t)n, &img);
   if (e != hipSuccess) {
-    if (e != hipErrorOutOfMemory) *err = e;
+    if (e == hipErrorOutOfMemory) be->refused = (size_t)n;
+    else *err = e;
     return nullptr;
   }
   const int rc = gemv_kimage_own(ttype)
@@ -714,6 +730,7 @@ void qhip_backend_free_linear(qhip_backend* be, qhip_linear* w) {
         (void)hipFree(it->second.p);
         be->placed -= it->second.bytes;
         it = be->images.erase(it);
+        be->refused = SIZE_MAX;
       } else {
         ++it;
       }
@@ -732,7 +749,8 @@ void qhip_backend_free_linear(qhip_backend* be, qhip_linear* w) {
 
 int qhip_backend_prepare_linear(qhip_backend* be, const qhip_linear* w) {
   if (!be || !valid_linear(w)) return (int)hipErrorInvalidValue;
-  // a long prefill: whether any token count would use an image for this weight
+  be->refused = SIZE_MAX;
+  int rc = 0;
   const GemvArgs g1{w->ttype, w->dev, w->dev, nullptr, w->rows, w->cols, 1, w->row_bytes,
                     qhip_act_row_bytes(w->ttype, w->cols)};
   if (be->gemv_images_on && (gemv_image_preferred(g1) || gemv_kimage_preferred(g1))) {
@@ -741,10 +759,9 @@ int qhip_backend_prepare_linear(qhip_backend* be, const qhip_linear* w) {
     hipError_t e;
     const uint8_t* img = gimage_for(be, w->dev, w->ttype, w->rows, w->cols, w->row_bytes, &e);
     if (e != hipSuccess) return report("GEMV image", e);
-    if (!img) return QHIP_DECLINE;
+    if (!img) rc = QHIP_DECLINE;
   }
   // a few tokens (the fragment image) and a long prefill (the MMQ image)
-  int rc = 0;
   for (const int kind : {kImgFrag, kImgMmq}) {
     const GemvArgs g{w->ttype, w->dev, w->dev, nullptr, w->rows, w->cols, kind == kImgFrag ? 8 : 4096,
                      w->row_bytes, qhip_act_row_bytes(w->ttype, w->cols)};
@@ -812,6 +829,7 @@ void qhip_backend_free_scratch(qhip_backend* be) {
     be->placed -= b.second;
   }
   be->retired.clear();
+  be->refused = SIZE_MAX;
 }
 
 int qhip_backend_alloc_buf(qhip_backend* be, size_t len, float** d_out) {
@@ -819,7 +837,7 @@ int qhip_backend_alloc_buf(qhip_backend* be, size_t len, float** d_out) {
   const size_t bytes = len ? len * sizeof(float) : sizeof(float);
   if (over_budget(be, bytes)) return (int)budget_error(be, "allocBuf", bytes);
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, bytes);
+  hipError_t e = dev_alloc(&p, bytes);
   if (e != hipSuccess) return report("allocBuf", e);
   be->bufs.emplace_back(p, bytes);
   be->placed += bytes;

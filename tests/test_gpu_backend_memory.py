@@ -1,0 +1,42 @@
+"""GPU: the Exec mirror where device memory is short -- images that the card or
+the budget has no room for, and what is asked for after them."""
+import numpy as np
+import pytest
+import torch
+
+import pyoracle as po
+from qwen35_amd import _lib, ops, synth
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-5
+
+
+def rel_l2(got, want):
+    got, want = np.asarray(got, np.float64), np.asarray(want, np.float64)
+    return float(np.linalg.norm(got - want) / max(np.linalg.norm(want), 1e-30))
+
+
+@pytest.fixture
+def backend(gpu):
+    be = ops.Backend(0)
+    yield be
+    be.close()
+
+
+@pytest.mark.parametrize("tt", [po.TT_Q5_K, po.TT_Q3_K, po.TT_IQ4_XS])
+def test_refused_image_leaves_no_error(gpu, oracle, backend, tt):
+    """Images larger than the card are refused when the weight is prepared, and
+    the products that follow on this thread still succeed."""
+    rows, cols, few = 64, 5120, 40
+    w = synth.make_weight(tt, rows, cols, seed=61, tag=tt)
+    lin = backend.load_linear(tt, rows, cols, w)
+    # a handle alone: nothing is read through it, for no image is allocated
+    huge = _lib.QhipLinear(lin.dev, tt, 1 << 26, 17408, _lib.load().qhip_weight_row_bytes(tt, 17408))
+    placed = backend.mem_placed()
+    assert backend.prepare_linear(huge) == -1 and backend.mem_placed() == placed
+    for tokens in (1, few):
+        x = synth.make_act(cols, tokens, seed=62)
+        out = torch.empty((tokens, rows), device=gpu)
+        backend.matvec_batch_k(out, lin, torch.from_numpy(x).to(gpu), tokens)
+        assert rel_l2(out.cpu().numpy(), oracle.matvec(tt, w, x)) < TOL
+    assert backend.prepare_linear(lin) == 0  # a refusal is not kept against a smaller image
