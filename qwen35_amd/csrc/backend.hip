@@ -310,6 +310,13 @@ static bool act_room(const qhip_backend* be, size_t bytes) {
          (!capturing(be->stream) && !over_budget(be, be->graph_seen ? bytes : bytes - be->act_cap));
 }
 
+// The activation scratch at `bytes`, grown now if need be.  A product from an
+// image asks for it before the image: built first, the image could take the
+// last of the budget or of the card from the scratch.
+static bool act_ready(qhip_backend* be, size_t bytes) {
+  return be->act_cap >= bytes || (act_room(be, bytes) && ensure_act(be, bytes) == hipSuccess);
+}
+
 // memo family of the split activation the GEMV image reads: kFamSplit plus
 // its layout (gemv_image_layout; the other families are the activation
 // block sizes, 32 and 256)
@@ -421,7 +428,7 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
     // the 32-value 4-bit formats on larger matrices: split quantize + GEMV
     // from the weight's GEMV image
     const GemvArgs g1{ttype, wdev, x, out, rows, cols, 1, row_bytes, qhip_act_row_bytes(ttype, cols)};
-    if (gemv_image_preferred(g1)) {
+    if (gemv_image_preferred(g1) && act_ready(be, act_bytes_for(cols, 1))) {
       hipError_t ei;
       uint8_t* img = gimage_for(be, wdev, ttype, rows, cols, row_bytes, &ei);
       if (ei != hipSuccess) return report("GEMV image", ei);
@@ -431,8 +438,6 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
                         be->memo_fam == sfam && be->act;
         if (be->memo_on) (hs ? be->memo_hits : be->memo_misses)++;
         if (!hs) {
-          const hipError_t ea = ensure_act(be, act_bytes_for(cols, 1));
-          if (ea != hipSuccess) return report("activation scratch", ea);
           memo_clear(be);
           const int rq = qhip_launch_quantize_act_image(ttype, x, be->act, cols, 1, be->stream);
           if (rq) return report("quantize", (hipError_t)rq);
@@ -453,7 +458,7 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
   uint8_t* kimg = nullptr;
   if (k == 1 && be->gemv_images_on) {
     const GemvArgs gk{ttype, wdev, x, out, rows, cols, 1, row_bytes, qhip_act_row_bytes(ttype, cols)};
-    if (gemv_kimage_preferred(gk)) {
+    if (gemv_kimage_preferred(gk) && act_ready(be, act_bytes_for(cols, 1))) {
       hipError_t ei;
       kimg = gimage_for(be, wdev, ttype, rows, cols, row_bytes, &ei);
       if (ei != hipSuccess) return report("GEMV image", ei);
@@ -464,7 +469,7 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
     // (whole groups of 32 tokens: where the scratch has room for the tokens'
     // Q8_K rows only, the product runs on those)
     const GemvArgs gp{ttype, wdev, x, out, rows, cols, k, row_bytes, qhip_act_row_bytes(ttype, cols)};
-    if (planes_preferred(gp) && act_room(be, (size_t)planes_act_bytes(cols, k))) {
+    if (planes_preferred(gp) && act_ready(be, (size_t)planes_act_bytes(cols, k))) {
       hipError_t e;
       const void* img = image_for(be, wdev, ttype, rows, cols, kImgMmq, &e);
       if (e != hipSuccess) return report("MMQ image", e);
@@ -473,8 +478,6 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
                         be->memo_fam == kFamMmq && be->act;
         if (be->memo_on) (hm ? be->memo_hits : be->memo_misses)++;
         if (!hm) {
-          e = ensure_act(be, (size_t)planes_act_bytes(cols, k));
-          if (e != hipSuccess) return report("activation scratch", e);
           memo_clear(be);
           e = launch_quantize_mmq_act(x, be->act, cols, k, be->stream);
           if (e != hipSuccess) return report("quantize", e);

@@ -40,3 +40,31 @@ def test_refused_image_leaves_no_error(gpu, oracle, backend, tt):
         backend.matvec_batch_k(out, lin, torch.from_numpy(x).to(gpu), tokens)
         assert rel_l2(out.cpu().numpy(), oracle.matvec(tt, w, x)) < TOL
     assert backend.prepare_linear(lin) == 0  # a refusal is not kept against a smaller image
+
+
+# a prompt from the plane image, and one token from a GEMV image
+@pytest.mark.parametrize("tt,rows,cols,tokens", [(po.TT_Q3_K, 300, 1024, 140), (po.TT_Q6_K, 300, 1024, 140),
+                                                 (po.TT_Q5_K, 300, 9728, 1), (po.TT_IQ4_NL, 2049, 5120, 1)])
+def test_image_leaves_room_for_the_activations(gpu, oracle, backend, tt, rows, cols, tokens):
+    """A budget that holds the image or the activations, not both: the image is
+    not built and the product runs from the GGUF rows."""
+    w = synth.make_weight(tt, rows, cols, seed=63, tag=tt)
+    x = synth.make_act(cols, tokens, seed=64)
+    xd, out = torch.from_numpy(x).to(gpu), torch.empty((tokens, rows), device=gpu)
+    lin = backend.load_linear(tt, rows, cols, w)
+    base = backend.mem_placed()
+    assert backend.prepare_linear(lin) == 0
+    image = backend.mem_placed() - base
+    assert image > 0
+    again = ops.Backend(0)
+    try:
+        lin = again.load_linear(tt, rows, cols, w)
+        again.set_mem_budget(again.mem_placed() + image + 512)
+        for _ in range(2):
+            out.fill_(float("nan"))
+            again.matvec_batch_k(out, lin, xd, tokens)
+            at = np.unique(np.r_[0:min(rows, 300), rows - 1])
+            want = oracle.matvec(tt, np.ascontiguousarray(w.reshape(rows, -1)[at]), x)
+            assert rel_l2(out.cpu().numpy()[:, at], want) < TOL
+    finally:
+        again.close()
