@@ -428,11 +428,15 @@ int qhip_backend_prepare_linear(qhip_backend *be, const qhip_linear *w);
 int qhip_backend_set_mmq_images(qhip_backend *be, int on);
 /* GEMV images on (default) or off; off, matvec never builds or reads one. */
 int qhip_backend_set_gemv_images(qhip_backend *be, int on);
-/* Cap on the device bytes this backend places (uploaded weights, MMQ images,
+/* Cap on the device bytes this backend places (uploaded weights, images,
  * scratch, workspaces, allocBuf regions); 0 = no cap (the default).
  * QWEN35_CUDA_MAX_DEV_MIB of src/backend_cuda.zig:1754-1760 as an argument:
- * a load or buffer past it fails with hipErrorOutOfMemory and a message; an
- * MMQ image past it is simply not built.  mem_placed: bytes counted so far. */
+ * an image past it is simply not built, and a load, scratch or buffer that
+ * does not fit beside the images gets their room (the largest MMQ images
+ * first, then the GEMV images; the products then read the GGUF bytes), on a
+ * full card as under a cap.  Not once a launch was captured into a graph, which
+ * may read them.  What does not fit without them fails with
+ * hipErrorOutOfMemory and a message.  mem_placed: bytes counted so far. */
 int qhip_backend_set_mem_budget(qhip_backend *be, size_t bytes);
 size_t qhip_backend_mem_placed(const qhip_backend *be);
 int qhip_backend_alloc_scratch(qhip_backend *be, int max_cols);

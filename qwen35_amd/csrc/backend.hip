@@ -90,9 +90,10 @@ struct qhip_backend {
   bool gemv_images_on = true;
   // Device-memory budget (QWEN35_CUDA_MAX_DEV_MIB, backend_cuda.zig:1754-1760,
   // as an argument): bytes this backend places on the device -- uploaded
-  // weights, MMQ images, scratch, workspaces, allocBuf regions.  0 = no cap.
-  // A load past the budget fails; an image past it is not built (the prefill
-  // then runs the tile MMQ on the GGUF bytes).
+  // weights, images, scratch, workspaces, allocBuf regions.  0 = no cap.
+  // An image past the budget is not built (the product then reads the GGUF
+  // bytes), and images are given back for a load, scratch or region that would
+  // not fit beside them; one that does not fit without them fails.
   size_t budget = 0;
   size_t placed = 0;  // bytes counted against the budget
   // The smallest image that the card had no memory for, until prepare_linear
@@ -169,9 +170,55 @@ static hipError_t dev_alloc(void** p, size_t bytes) {
   return e;
 }
 
+static bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+}
+
+// Give one image's memory back: the largest plane or fragment image, or, when
+// there is none, all GEMV images (one arena).  Products then read the GGUF
+// rows.  Images are copies that only make products faster, so they make way
+// for what a call cannot do without: weights, scratch, allocBuf regions.  Not
+// once a graph was captured, which may read them.
+static bool give_back_image(qhip_backend* be) {
+  if (be->graph_seen || capturing(be->stream)) return false;
+  if (be->images.empty() && be->img_arena.empty()) return false;
+  (void)hipStreamSynchronize(be->stream);
+  if (!be->images.empty()) {
+    auto big = be->images.begin();
+    for (auto it = be->images.begin(); it != be->images.end(); ++it)
+      if (it->second.bytes > big->second.bytes) big = it;
+    (void)hipFree(big->second.p);
+    be->placed -= big->second.bytes;
+    be->images.erase(big);
+    return true;
+  }
+  for (auto& c : be->img_arena) {
+    (void)hipFree(c.base);
+    be->placed -= c.used;
+  }
+  be->img_arena.clear();
+  be->gimages.clear();
+  return true;
+}
+
+// Whether the budget holds `more` bytes, images given back for them if need be.
+static bool make_room(qhip_backend* be, size_t more) {
+  while (over_budget(be, more))
+    if (!give_back_image(be)) return false;
+  return true;
+}
+
+// dev_alloc for what a call cannot do without.
+static hipError_t dev_alloc_must(qhip_backend* be, void** p, size_t bytes) {
+  hipError_t e = dev_alloc(p, bytes);
+  while (e == hipErrorOutOfMemory && give_back_image(be)) e = dev_alloc(p, bytes);
+  return e;
+}
+
 static hipError_t arena_alloc(qhip_backend* be, size_t bytes, uint8_t** out) {
   bytes = (bytes + kAlign - 1) / kAlign * kAlign;
-  if (over_budget(be, bytes)) return budget_error(be, "weight upload", bytes);
+  if (!make_room(be, bytes)) return budget_error(be, "weight upload", bytes);
   if (!be->arena.empty()) {
     auto& c = be->arena.back();
     if (c.size - c.used >= bytes) {
@@ -185,17 +232,12 @@ static hipError_t arena_alloc(qhip_backend* be, size_t bytes, uint8_t** out) {
   size_t sz = bytes > kArenaChunk ? bytes : kArenaChunk;
   if (be->budget && sz > be->budget - be->placed) sz = bytes > be->budget - be->placed ? bytes : be->budget - be->placed;
   void* p = nullptr;
-  hipError_t e = dev_alloc(&p, sz);
+  hipError_t e = dev_alloc_must(be, &p, sz);
   if (e != hipSuccess) return e;
   be->arena.push_back({(uint8_t*)p, sz, bytes});
   be->placed += bytes;
   *out = (uint8_t*)p;
   return hipSuccess;
-}
-
-static bool capturing(hipStream_t s) {
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
 }
 
 // Give up a scratch buffer that is being replaced by a larger one: freed now,
@@ -223,7 +265,7 @@ static size_t grown_size(const qhip_backend* be, size_t cap, size_t bytes) {
 
 static hipError_t ensure_act(qhip_backend* be, size_t bytes) {
   if (be->act_cap >= bytes) return hipSuccess;
-  if (over_budget(be, be->graph_seen ? bytes : bytes - be->act_cap))
+  if (!make_room(be, be->graph_seen ? bytes : bytes - be->act_cap))
     return budget_error(be, "activation scratch", bytes - be->act_cap);
   bytes = grown_size(be, be->act_cap, bytes);
   release_buffer(be, be->act, be->act_cap);
@@ -231,7 +273,7 @@ static hipError_t ensure_act(qhip_backend* be, size_t bytes) {
   be->act_cap = 0;
   memo_clear(be);
   void* p = nullptr;
-  hipError_t e = dev_alloc(&p, bytes);
+  hipError_t e = dev_alloc_must(be, &p, bytes);
   if (e != hipSuccess) return e;
   be->act = (uint8_t*)p;
   be->act_cap = bytes;
@@ -239,16 +281,19 @@ static hipError_t ensure_act(qhip_backend* be, size_t bytes) {
   return hipSuccess;
 }
 
-static hipError_t ensure_skwork(qhip_backend* be, size_t bytes) {
+// must: the launch cannot do without it (the MMQ runs unsplit; its caller may
+// hold an image, so none is given back for it)
+static hipError_t ensure_skwork(qhip_backend* be, size_t bytes, bool must) {
   if (be->skwork_cap >= bytes) return hipSuccess;
-  if (over_budget(be, be->graph_seen ? bytes : bytes - be->skwork_cap))
+  const size_t more = be->graph_seen ? bytes : bytes - be->skwork_cap;
+  if (must ? !make_room(be, more) : over_budget(be, more))
     return budget_error(be, "split-K workspace", bytes - be->skwork_cap);
   bytes = grown_size(be, be->skwork_cap, bytes);
   release_buffer(be, be->skwork, be->skwork_cap);
   be->skwork = nullptr;
   be->skwork_cap = 0;
   void* p = nullptr;
-  hipError_t e = dev_alloc(&p, bytes);
+  hipError_t e = must ? dev_alloc_must(be, &p, bytes) : dev_alloc(&p, bytes);
   if (e != hipSuccess) return e;
   // the counters start at zero; a fill kernel on the backend's stream orders
   // it before the first split launch
@@ -492,7 +537,7 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
         // a launch that does not fit runs unsplit)
         const long need = planes_work_bytes(rows, cols, k);
         if (need > 0 && (size_t)need > be->skwork_cap && !capturing(be->stream)) {
-          e = ensure_skwork(be, (size_t)need);
+          e = ensure_skwork(be, (size_t)need, false);
           if (e != hipSuccess && e != hipErrorOutOfMemory) return report("split-K workspace", e);
         }
         return report("matvec", launch_mmq_planes(ttype, img, be->act, out, rows, cols, k, be->skwork,
@@ -521,7 +566,7 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
       int rc;
       if (split) {
         const long wb = gemv_splitk_work_bytes(rows, cols);
-        const hipError_t ew = ensure_skwork(be, (size_t)wb);
+        const hipError_t ew = ensure_skwork(be, (size_t)wb, true);
         if (ew != hipSuccess) return report("split-K workspace", ew);
         rc = qhip_launch_quantize_mul_mat_vec_split(wdev, x, xq_out, out, rows, cols, ttype, 0, 0, 0, be->skwork,
                                                     (long)be->skwork_cap, be->stream);
@@ -566,7 +611,7 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
   // only (under capture a launch that does not fit runs unsplit)
   const long need = mul_mat_work_bytes(g);
   if (need > 0 && (size_t)need > be->skwork_cap && !capturing(be->stream)) {
-    e = ensure_skwork(be, (size_t)need);
+    e = ensure_skwork(be, (size_t)need, false);
     if (e != hipSuccess && e != hipErrorOutOfMemory) return report("split-K workspace", e);
   }
   void* work = be->skwork;
@@ -838,9 +883,9 @@ void qhip_backend_free_scratch(qhip_backend* be) {
 int qhip_backend_alloc_buf(qhip_backend* be, size_t len, float** d_out) {
   if (!be || !d_out) return (int)hipErrorInvalidValue;
   const size_t bytes = len ? len * sizeof(float) : sizeof(float);
-  if (over_budget(be, bytes)) return (int)budget_error(be, "allocBuf", bytes);
+  if (!make_room(be, bytes)) return (int)budget_error(be, "allocBuf", bytes);
   void* p = nullptr;
-  hipError_t e = dev_alloc(&p, bytes);
+  hipError_t e = dev_alloc_must(be, &p, bytes);
   if (e != hipSuccess) return report("allocBuf", e);
   be->bufs.emplace_back(p, bytes);
   be->placed += bytes;

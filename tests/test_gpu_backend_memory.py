@@ -1,5 +1,7 @@
 """GPU: the Exec mirror where device memory is short -- images that the card or
 the budget has no room for, and what is asked for after them."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -68,3 +70,53 @@ def test_image_leaves_room_for_the_activations(gpu, oracle, backend, tt, rows, c
             assert rel_l2(out.cpu().numpy()[:, at], want) < TOL
     finally:
         again.close()
+
+
+def test_images_make_way_for_later_weights(gpu, oracle, backend):
+    """Under a budget that the first weight's images fill, a second weight, a
+    scratch and a buffer are still placed; products read what is left."""
+    tt, rows, cols, tokens = po.TT_Q5_K, 2048, 5120, 40
+    ws = [synth.make_weight(tt, rows, cols, seed=65 + i, tag=tt) for i in range(3)]
+    budget = 9 * rows * cols // 2  # six weights' bytes, or one weight and its images
+    backend.set_mem_budget(budget)
+    lins = [backend.load_linear(tt, rows, cols, ws[0])]
+    assert backend.prepare_linear(lins[0]) == 0
+    assert backend.mem_placed() > 4 * rows * cols  # no room beside them
+    lins += [backend.load_linear(tt, rows, cols, w) for w in ws[1:]]
+    buf = ctypes.c_void_p()
+    assert backend.lib.qhip_backend_alloc_buf(backend._h, rows * cols // 8, ctypes.byref(buf)) == 0 and buf.value
+    for lin, w in zip(lins, ws):
+        for k in (1, tokens):
+            x = synth.make_act(cols, k, seed=68)
+            out = torch.empty((k, rows), device=gpu)
+            backend.matvec_batch_k(out, lin, torch.from_numpy(x).to(gpu), k)
+            assert rel_l2(out.cpu().numpy(), oracle.matvec(tt, w, x)) < TOL
+    assert backend.mem_placed() <= budget
+
+
+def test_captured_images_stay(gpu, oracle, backend):
+    """A graph captured from an image keeps it: a load that would need its room
+    is refused, and the graph replays on."""
+    tt, rows, cols = po.TT_Q5_K, 512, 5120
+    w = synth.make_weight(tt, rows, cols, seed=69, tag=tt)
+    lin = backend.load_linear(tt, rows, cols, w)
+    assert backend.prepare_linear(lin) == 0
+    x, out = torch.empty((1, cols), device=gpu), torch.empty((1, rows), device=gpu)
+    side = torch.cuda.Stream()
+    backend.set_stream(side)
+    backend.matvec(out, lin, x)  # the scratch
+    side.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        backend.matvec(out, lin, x)
+    placed = backend.mem_placed()
+    backend.set_mem_budget(placed + 1024)
+    with pytest.raises(Exception):
+        backend.load_linear(tt, rows, cols, w)
+    assert backend.mem_placed() == placed
+    for i in range(3):
+        xi = synth.make_act(cols, 1, seed=70 + i)
+        x.copy_(torch.from_numpy(xi))
+        g.replay()
+        torch.cuda.synchronize()
+        assert rel_l2(out.cpu().numpy(), oracle.matvec(tt, w, xi)) < TOL
