@@ -21,6 +21,8 @@
 #include "qhip_device.hpp"
 #include "qhip_internal.hpp"
 
+#include "../../include/qwen35_hip.h"
+
 namespace qhip {
 
 template <int TT, int NT, int NR, bool IMG = false, int WPB = 4>
@@ -1067,6 +1069,19 @@ static void fused_default_shape(const GemvArgs& g, int& team, int& nr, int& wgs)
   }
   team = best;
   nr = 1;
+}
+
+// Whether the fused launch's workgroups run at once (1024 threads: one per CU).  A
+// grid a little past that takes a second round: Q8_0 [12800, 2560] (267 workgroups)
+// 13.8 us against 11.4 from the GEMV image, [5120, 5120] (320) 12.7 / 10.2, [10240,
+// 3072] (320) 12.5 / 11.4; but [8192, 3584] (256) 8.9 / 13.5, [7168, 4608] (224)
+// 11.1 / 15.1, [31744, 1024] (248) 9.3 / 10.4.
+bool gemv_fused_one_round(const GemvArgs& g) {
+  int team, nr, wgs;
+  fused_default_shape(g, team, nr, wgs);
+  const long waves = ((long)g.rows + 64 / team - 1) / (64 / team);
+  const int cus = qhip_gpu_cu_count();
+  return (waves + wgs / 64 - 1) / (wgs / 64) <= (cus > 0 ? cus : 256);
 }
 
 // Fused quantize + GEMV against separate quantize and GEMV launches, measured

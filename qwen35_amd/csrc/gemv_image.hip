@@ -341,11 +341,15 @@ static hipError_t launch_img_tt(const GemvArgs& g, int T, int P, int nr, hipStre
 // (fused 12.0), Q8_0 14.4 vs 18.7 (16.3); at [8192, 4096] the two meet (IQ4_NL
 // 8.9 / fused 9.0, Q8_0 11.2 / 10.5, Q4_0 8.7 / 8.1).  Below 2^25 weights the
 // fused launch wins (Q8_0 [9728, 2560] 9.3 us against 10.0 from the image,
-// IQ4_NL [4096, 4096] 6.2 against 7.2, [6144, 1024] 4.4 against 5.6); rows too
-// wide for it read the image from 2^23.
+// IQ4_NL [4096, 4096] 6.2 against 7.2, [6144, 1024] 4.4 against 5.6) where its
+// grid runs in one round (gemv_fused_one_round); rows too wide for it read the
+// image from 2^23.
+bool gemv_image_pays(const GemvArgs& g) {
+  return g.tokens == 1 && gemv_image_format(g.ttype) && gemv_image_width(g.cols) && (long)g.rows * g.cols > (1L << 23);
+}
 bool gemv_image_preferred(const GemvArgs& g) {
-  return g.tokens == 1 && gemv_image_format(g.ttype) && gemv_image_width(g.cols) &&
-         (long)g.rows * g.cols > (1L << 23) && (!gemv_fused_preferred(g) || (long)g.rows * g.cols >= (1L << 25));
+  return gemv_image_pays(g) &&
+         (!gemv_fused_preferred(g) || (long)g.rows * g.cols >= (1L << 25) || !gemv_fused_one_round(g));
 }
 
 // ---- K-quant GEMV image (Q4_K, Q6_K) --------------------------------------------

@@ -48,6 +48,7 @@ constexpr long kFusedMaxLds = 64 * 1024;
 bool gemv_fused_fits(int ttype, int cols);
 // whether the fused launch beats quantize + GEMV for this shape (measured rule)
 bool gemv_fused_preferred(const GemvArgs& g);
+bool gemv_fused_one_round(const GemvArgs& g);
 // team / nr / wgs (workgroup threads: 256, or 512 / 1024 with nr <= 2) 0 = pick
 hipError_t launch_gemv_fused(const GemvArgs& g, const float* x, void* xq_out, int team, int nr, int wgs,
                              hipStream_t s);
@@ -122,7 +123,9 @@ hipError_t launch_quantize_act_image(int ttype, const float* x, void* out, int c
 // g.w = the image, g.xq = one token's split activation; nr rows per team (1,
 // 2; 0 = pick)
 hipError_t launch_gemv_image(const GemvArgs& g, int nr, hipStream_t s);
-// whether quantize + image GEMV beats the GGUF-layout launches (measured rule)
+// whether quantize + image GEMV beats quantize + GGUF-row GEMV, and whether it
+// beats the one-launch form as well (measured rules)
+bool gemv_image_pays(const GemvArgs& g);
 bool gemv_image_preferred(const GemvArgs& g);
 // K-quant GEMV image (Q4_K, Q6_K; KImg in qhip_device.hpp): the same bytes
 // per row, read by launch_gemv / launch_gemv_fused / launch_gemv_splitk when
