@@ -402,22 +402,21 @@ int qhip_backend_wrap_linear(qhip_backend *be, int ttype, int rows, int cols, co
 void qhip_backend_free_linear(qhip_backend *be, qhip_linear *w);
 /* Build what this weight's products use beyond its GGUF bytes now, at load
  * time, instead of inside the first matvec: the GEMV image of an IQ4_NL /
- * Q4_0 / Q8_0 weight large enough for the decode matvec to read it (past 2^23
- * weights, 2^25 where the one-launch quantize + GEMV takes the shape), or of a
- * Q6_K, Q5_K or Q2_K weight whose decode matvec quantizes separately (widths
- * above 4096, or more than 32768 rows) or a Q3_K weight of width 2560 or more and
- * more than 2^23 values (Q5_K and Q3_K: none narrower than 2560, Q2_K 4096;
- * the GGUF bytes once more, Q3_K 1.04x and Q5_K 1.02x; built in
- * load order, so adjacent weights get adjacent images and matvecPair stays one
- * launch), the fragment image of a Q6_K, Q5_K or Q4_K weight with rows * cols >=
- * 2^23 (qhip_launch_wd_prepare, the GGUF bytes once more; matvec_batch_k reads it
- * from 2 tokens, Q6_K up to 64, on rows below 12288 to 96, Q5_K to 128) or of a
- * Q8_0 weight with cols <= 1024 (from
- * 6 tokens) and the plane image of the other super-block formats' and Q6_K's
- * prompts (Q6_K, IQ4_XS and the IQ3 formats 2.02 bytes a weight, Q5_K 2.16,
- * Q3_K 1.02, Q2_K 1.16; read past the fragment image's tokens, from 65 where
- * there is none, Q3_K from 25, IQ4_XS and the
- * IQ3 formats from 129).
+ * Q4_0 / Q8_0 weight past 2^23 weights, of a Q6_K, Q5_K or Q2_K weight whose
+ * decode matvec, alone or as half of a matvecPair, quantizes separately (widths
+ * above 4096, or more than 32768 rows) or of a Q3_K weight of width 2560 or more
+ * that alone or as half of a pair has more than 2^23 values (Q5_K and Q3_K: none
+ * narrower than 2560, Q2_K 4096; the GGUF bytes once more, Q3_K 1.04x and Q5_K
+ * 1.02x; built in load order, so adjacent weights get adjacent images and
+ * matvecPair stays one launch), the fragment image of a Q6_K, Q5_K or Q4_K weight
+ * with rows * cols >= 2^23 (qhip_launch_wd_prepare, the GGUF bytes once more;
+ * matvec_batch_k reads it from 2 tokens, Q6_K up to 64, on rows below 12288 to
+ * 96, Q5_K to 128) or of a Q8_0 weight with cols <= 1024 (from 6 tokens) and the
+ * plane image of the other super-block formats' and Q6_K's prompts (Q6_K,
+ * IQ4_XS and the IQ3 formats 2.02 bytes a weight, Q5_K 2.16, Q3_K 1.02, Q2_K
+ * 1.16; read past the fragment image's tokens, from 65 where there is none, Q3_K
+ * from 25, IQ4_XS and the IQ3 formats from 129).  A program that decodes only
+ * saves the MMQ images' time and room with qhip_backend_set_mmq_images(be, 0).
  * 0 = built or nothing to build; QHIP_DECLINE = not all built (images off, or
  * past the memory budget): the products then read the GGUF bytes.
  * No reference counterpart (its CUDA kernels decode the GGUF blocks in every

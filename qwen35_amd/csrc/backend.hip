@@ -10,6 +10,7 @@
 #include "qhip_internal.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
@@ -470,10 +471,13 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
   // 256-value super-blocks (backend_cpu.zig:42-50 actFamily)
   const int fam = qhip_quant_act_block_elems(ttype);
   if (k == 1 && be->gemv_images_on) {
-    // the 32-value 4-bit formats on larger matrices: split quantize + GEMV
-    // from the weight's GEMV image
+    // IQ4_NL, Q4_0 and Q8_0 on larger matrices: split quantize + GEMV from the
+    // weight's GEMV image.  The one-launch form is out where x is not aligned
+    // for it; with the memo on it would quantize once for this product only:
+    // the next one of x would read the GGUF rows.
     const GemvArgs g1{ttype, wdev, x, out, rows, cols, 1, row_bytes, qhip_act_row_bytes(ttype, cols)};
-    if (gemv_image_preferred(g1) && act_ready(be, act_bytes_for(cols, 1))) {
+    const bool only = be->memo_on || ((uintptr_t)x & 15u);
+    if ((only ? gemv_image_pays(g1) : gemv_image_preferred(g1)) && act_ready(be, act_bytes_for(cols, 1))) {
       hipError_t ei;
       uint8_t* img = gimage_for(be, wdev, ttype, rows, cols, row_bytes, &ei);
       if (ei != hipSuccess) return report("GEMV image", ei);
@@ -801,7 +805,11 @@ int qhip_backend_prepare_linear(qhip_backend* be, const qhip_linear* w) {
   int rc = 0;
   const GemvArgs g1{w->ttype, w->dev, w->dev, nullptr, w->rows, w->cols, 1, w->row_bytes,
                     qhip_act_row_bytes(w->ttype, w->cols)};
-  if (be->gemv_images_on && (gemv_image_preferred(g1) || gemv_kimage_preferred(g1))) {
+  // matvec_pair multiplies two adjacent weights as one of twice the rows
+  GemvArgs g2 = g1;
+  if (w->rows <= INT_MAX / 2) g2.rows = 2 * w->rows;
+  if (be->gemv_images_on && (gemv_image_pays(g1) || gemv_image_preferred(g2) || gemv_kimage_preferred(g1) ||
+                             gemv_kimage_preferred(g2))) {
     // a decode matvec: the GEMV image
     if (capturing(be->stream)) return (int)hipErrorStreamCaptureUnsupported;
     hipError_t e;

@@ -1,5 +1,6 @@
-"""GPU: when a one-token product of the Exec mirror reads its weight's GEMV
-image."""
+"""GPU: when a one-token product of the Exec mirror reads its weight's GEMV image
+-- as one weight and as half of an adjacent pair, with the activation memo on,
+and for an x that the one-launch form does not take."""
 import numpy as np
 import pytest
 import torch
@@ -21,6 +22,77 @@ def backend(gpu):
     be = ops.Backend(0)
     yield be
     be.close()
+
+
+def load_pair(be, tt, rows, cols, seed):
+    w = synth.make_weight(tt, 2 * rows, cols, seed=seed, tag=tt).reshape(2 * rows, -1)
+    return w, [be.load_linear(tt, rows, cols, part) for part in (w[:rows], w[rows:])]
+
+
+# every weight alone takes the one-launch form (Q3_K: too small for an image),
+# the pair an image
+@pytest.mark.parametrize("tt,rows,cols", [(po.TT_Q8_0, 4160, 4096), (po.TT_IQ4_NL, 4160, 4096),
+                                          (po.TT_Q5_K, 16400, 2560), (po.TT_Q3_K, 1792, 2560)])
+def test_prepared_pair_is_captured_from_its_images(gpu, oracle, backend, tt, rows, cols):
+    w, (a, b) = load_pair(backend, tt, rows, cols, seed=71)
+    assert backend.lib.qhip_backend_alloc_scratch(backend._h, cols) == 0
+    assert backend.prepare_linear(a) == 0 and backend.prepare_linear(b) == 0
+    placed = backend.mem_placed()
+    x, out = torch.empty(cols, device=gpu), torch.empty(2 * rows, device=gpu)
+    side = torch.cuda.Stream()
+    backend.set_stream(side)
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=side):
+        backend.matvec_pair(out, a, b, x)
+    backend.set_stream(torch.cuda.current_stream())
+    eager = torch.empty_like(out)
+    at = np.unique(np.linspace(0, 2 * rows - 1, 200).astype(int))
+    for i in range(3):
+        xi = synth.make_act(cols, 1, seed=72 + i)
+        x.copy_(torch.from_numpy(xi[0]))
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert rel_l2(out.cpu().numpy()[at], oracle.matvec(tt, np.ascontiguousarray(w[at]), xi)[0]) < TOL
+        backend.matvec_pair(eager, a, b, x)
+        assert torch.equal(out, eager)  # the same launch, so the graph reads the images too
+    assert backend.mem_placed() == placed  # nothing was left to build
+
+
+@pytest.mark.parametrize("tt", [po.TT_Q8_0, po.TT_IQ4_NL])
+def test_memo_and_unaligned_x_read_the_image(gpu, oracle, backend, tt):
+    rows, cols = 3300, 2560  # above 2^23 weights, where the one-launch form is the faster of the two
+    w = synth.make_weight(tt, rows, cols, seed=75, tag=tt)
+    lin = backend.load_linear(tt, rows, cols, w)
+    base = backend.mem_placed()
+    assert backend.prepare_linear(lin) == 0
+    assert backend.mem_placed() > base
+    x = synth.make_act(cols, 1, seed=76)
+    buf = torch.empty(cols + 4, device=gpu)
+    outs = {}
+    for shift in (0, 1):  # floats past a 16-byte boundary
+        xd = buf[shift:shift + cols]
+        xd.copy_(torch.from_numpy(x[0]))
+        for memo in (False, True):
+            backend.set_act_memo(memo)
+            for again in range(2):
+                out = torch.empty(rows, device=gpu)
+                backend.matvec(out, lin, xd)
+                outs[shift, memo, again] = out
+    want = oracle.matvec(tt, w, x)[0]
+    for out in outs.values():
+        assert rel_l2(out.cpu().numpy(), want) < TOL
+    image = outs[1, False, 0]
+    for key, out in outs.items():
+        if key[0] == 1 or key[1]:
+            assert torch.equal(out, image), key
+    hits, misses = backend.act_stats()
+    assert (hits, misses) == (2, 2)  # per x, the second product reuses the first one's activation
+    backend.set_act_memo(False)
+    backend.set_gemv_images(False)
+    backend.matvec(image, lin, buf[1:1 + cols])
+    assert not torch.equal(image, outs[0, True, 0])  # the rows are summed in another order
 
 
 # one round of the one-launch form's workgroups | a little past it
