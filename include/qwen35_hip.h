@@ -469,7 +469,10 @@ int qhip_backend_sync(qhip_backend *be);
  * x pointer, width, token count and activation family (Q8_0 or Q8_K) match
  * the last quantization reuses the quantized rows in the scratch instead of
  * quantizing again (q/k/v of one hidden state, Q4_K and Q6_K weights of one
- * x, the halves of a non-adjacent matvecPair).  Off by default.  The caller
+ * x, the halves of a non-adjacent matvecPair); a prompt's activation image
+ * (prepare_linear: the plane-image products) is remembered beside them, in a
+ * scratch of its own that alloc_scratch_k reserves while the memo is on.  Off
+ * by default.  The caller
  * must call qhip_backend_act_invalidate after anything writes into a buffer
  * a matvec may read again (the reference clears at the same points,
  * backend_cuda.zig:6250-6254: rmsnorm, l2norm, add_resid, copy_range,

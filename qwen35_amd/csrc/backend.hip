@@ -101,14 +101,23 @@ struct qhip_backend {
   // asks again or this backend gives memory back: a matvec without its image
   // does not try the allocation anew on every call.
   size_t refused = SIZE_MAX;
-  // What `act` holds (backend_cuda.zig:3425-3448 actQValid/actQMark): the
-  // source pointer, width, token count and activation family of the last
+  // What `act` and `pact` hold (backend_cuda.zig:3425-3448 actQValid/actQMark):
+  // the source pointer, width, token count and activation family of the last
   // quantization, so a second matvec of the same x skips its quantize.
   // Off unless enabled; cleared by step_begin, act_invalidate, set_stream and
   // a scratch reallocation.
   bool memo_on = false;
-  const float* memo_src = nullptr;
-  int memo_cols = 0, memo_k = 0, memo_fam = -1;
+  struct Memo {
+    const float* src = nullptr;
+    int cols = 0, k = 0, fam = -1;
+    bool holds(const float* x, int c, int n, int f) const { return src == x && cols == c && k == n && fam == f; }
+  };
+  Memo memo, pmemo;
+  // With the memo on, a scratch of its own for the activation image of a
+  // prompt: the products of one x of a mixed recipe (Q4_K reads Q8_K rows, Q6_K
+  // the image) would evict each other's quantization from `act`.
+  uint8_t* pact = nullptr;
+  size_t pact_cap = 0;
   unsigned long long memo_hits = 0, memo_misses = 0;
   // Device timing of the slots (the Exec profiling slots, backend.zig:500-514;
   // the reference's per-type device table, backend_cuda.zig:6647): an event
@@ -145,9 +154,8 @@ struct qhip_backend {
 };
 
 static void memo_clear(qhip_backend* be) {
-  be->memo_src = nullptr;
-  be->memo_cols = be->memo_k = 0;
-  be->memo_fam = -1;
+  be->memo = {};
+  be->pmemo = {};
 }
 
 static constexpr size_t kArenaChunk = size_t(1) << 30;  // 1 GiB
@@ -272,7 +280,7 @@ static hipError_t ensure_act(qhip_backend* be, size_t bytes) {
   release_buffer(be, be->act, be->act_cap);
   be->act = nullptr;
   be->act_cap = 0;
-  memo_clear(be);
+  be->memo = {};
   void* p = nullptr;
   hipError_t e = dev_alloc_must(be, &p, bytes);
   if (e != hipSuccess) return e;
@@ -361,6 +369,24 @@ static bool act_room(const qhip_backend* be, size_t bytes) {
 // last of the budget or of the card from the scratch.
 static bool act_ready(qhip_backend* be, size_t bytes) {
   return be->act_cap >= bytes || (act_room(be, bytes) && ensure_act(be, bytes) == hipSuccess);
+}
+
+// The memo's own scratch for an activation image, or false: no room, and the
+// image shares the activation scratch.
+static bool pact_ready(qhip_backend* be, size_t bytes) {
+  if (be->pact_cap >= bytes) return true;
+  if (capturing(be->stream) || over_budget(be, be->graph_seen ? bytes : bytes - be->pact_cap)) return false;
+  bytes = grown_size(be, be->pact_cap, bytes);
+  release_buffer(be, be->pact, be->pact_cap);
+  be->pact = nullptr;
+  be->pact_cap = 0;
+  be->pmemo = {};
+  void* p = nullptr;
+  if (dev_alloc(&p, bytes) != hipSuccess) return false;
+  be->pact = (uint8_t*)p;
+  be->pact_cap = bytes;
+  be->placed += bytes;
+  return true;
 }
 
 // memo family of the split activation the GEMV image reads: kFamSplit plus
@@ -483,19 +509,13 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
       if (ei != hipSuccess) return report("GEMV image", ei);
       if (img) {
         const int sfam = kFamSplit + gemv_image_layout(ttype, cols);
-        const bool hs = be->memo_on && be->memo_src == x && be->memo_cols == cols && be->memo_k == 1 &&
-                        be->memo_fam == sfam && be->act;
+        const bool hs = be->memo_on && be->memo.holds(x, cols, 1, sfam);
         if (be->memo_on) (hs ? be->memo_hits : be->memo_misses)++;
         if (!hs) {
-          memo_clear(be);
+          be->memo = {};
           const int rq = qhip_launch_quantize_act_image(ttype, x, be->act, cols, 1, be->stream);
           if (rq) return report("quantize", (hipError_t)rq);
-          if (be->memo_on) {
-            be->memo_src = x;
-            be->memo_cols = cols;
-            be->memo_k = 1;
-            be->memo_fam = sfam;
-          }
+          if (be->memo_on) be->memo = {x, cols, 1, sfam};
         }
         return report("matvec", (hipError_t)qhip_launch_mul_mat_vec_image(img, be->act, out, rows, cols, ttype, 0,
                                                                            be->stream));
@@ -518,24 +538,23 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
     // (whole groups of 32 tokens: where the scratch has room for the tokens'
     // Q8_K rows only, the product runs on those)
     const GemvArgs gp{ttype, wdev, x, out, rows, cols, k, row_bytes, qhip_act_row_bytes(ttype, cols)};
-    if (planes_preferred(gp) && act_ready(be, (size_t)planes_act_bytes(cols, k))) {
+    const bool planes = planes_preferred(gp);
+    const size_t need_act = planes ? (size_t)planes_act_bytes(cols, k) : 0;
+    const bool own = planes && be->memo_on && pact_ready(be, need_act);
+    if (planes && (own || act_ready(be, need_act))) {
       hipError_t e;
       const void* img = image_for(be, wdev, ttype, rows, cols, kImgMmq, &e);
       if (e != hipSuccess) return report("MMQ image", e);
       if (img) {
-        const bool hm = be->memo_on && be->memo_src == x && be->memo_cols == cols && be->memo_k == k &&
-                        be->memo_fam == kFamMmq && be->act;
+        uint8_t* const xa = own ? be->pact : be->act;
+        qhip_backend::Memo& m = own ? be->pmemo : be->memo;
+        const bool hm = be->memo_on && m.holds(x, cols, k, kFamMmq);
         if (be->memo_on) (hm ? be->memo_hits : be->memo_misses)++;
         if (!hm) {
-          memo_clear(be);
-          e = launch_quantize_mmq_act(x, be->act, cols, k, be->stream);
+          m = {};
+          e = launch_quantize_mmq_act(x, xa, cols, k, be->stream);
           if (e != hipSuccess) return report("quantize", e);
-          if (be->memo_on) {
-            be->memo_src = x;
-            be->memo_cols = cols;
-            be->memo_k = k;
-            be->memo_fam = kFamMmq;
-          }
+          if (be->memo_on) m = {x, cols, k, kFamMmq};
         }
         // the split workspace is grown outside a capture only (under capture
         // a launch that does not fit runs unsplit)
@@ -544,13 +563,12 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
           e = ensure_skwork(be, (size_t)need, false);
           if (e != hipSuccess && e != hipErrorOutOfMemory) return report("split-K workspace", e);
         }
-        return report("matvec", launch_mmq_planes(ttype, img, be->act, out, rows, cols, k, be->skwork,
+        return report("matvec", launch_mmq_planes(ttype, img, xa, out, rows, cols, k, be->skwork,
                                                   (long)be->skwork_cap, be->stream));
       }
     }
   }
-  const bool hit = be->memo_on && be->memo_src == x && be->memo_cols == cols && be->memo_k == k &&
-                   be->memo_fam == fam && be->act;
+  const bool hit = be->memo_on && be->memo.holds(x, cols, k, fam);
   if (be->memo_on) (hit ? be->memo_hits : be->memo_misses)++;
   if (!hit && k == 1 && !kimg) {
     // one launch, the activation quantized inside the GEMV, where that is
@@ -564,7 +582,7 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
       if (be->memo_on) {
         const hipError_t ea = ensure_act(be, act_bytes_for(cols, 1));
         if (ea != hipSuccess) return report("activation scratch", ea);
-        memo_clear(be);
+        be->memo = {};
         xq_out = be->act;
       }
       int rc;
@@ -578,12 +596,7 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
         rc = qhip_launch_quantize_mul_mat_vec(wdev, x, xq_out, out, rows, cols, ttype, be->stream);
       }
       if (rc != QHIP_DECLINE) {
-        if (rc == 0 && xq_out) {
-          be->memo_src = x;
-          be->memo_cols = cols;
-          be->memo_k = 1;
-          be->memo_fam = fam;
-        }
+        if (rc == 0 && xq_out) be->memo = {x, cols, 1, fam};
         return report("matvec", (hipError_t)rc);
       }
     }
@@ -593,15 +606,10 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
   if (!hit) {
     e = ensure_act(be, act_bytes_for(cols, k));
     if (e != hipSuccess) return report("activation scratch", e);
-    memo_clear(be);
+    be->memo = {};
     rc = qhip_launch_quantize_act(ttype, x, be->act, cols, k, be->stream);
     if (rc) return report("quantize", (hipError_t)rc);
-    if (be->memo_on) {
-      be->memo_src = x;
-      be->memo_cols = cols;
-      be->memo_k = k;
-      be->memo_fam = fam;
-    }
+    if (be->memo_on) be->memo = {x, cols, k, fam};
   }
   GemvArgs g{ttype, wdev, be->act, out, rows, cols, k, row_bytes, qhip_act_row_bytes(ttype, cols)};
   if (kimg) {
@@ -860,7 +868,9 @@ int qhip_backend_alloc_scratch_k(qhip_backend* be, int max_cols, int k) {
   if (!be || max_cols <= 0 || k <= 0) return (int)hipErrorInvalidValue;
   // the activation image of a prompt is of whole 32-token groups
   const size_t rows = act_bytes_for(max_cols, k), groups = act_bytes_for(max_cols, (k + 31) / 32 * 32);
-  return report("scratch", ensure_act(be, k > 16 && act_room(be, groups) ? groups : rows));
+  const int rc = report("scratch", ensure_act(be, k > 16 && act_room(be, groups) ? groups : rows));
+  if (rc == 0 && be->memo_on && k > 16) (void)pact_ready(be, groups);
+  return rc;
 }
 
 void qhip_backend_free_scratch(qhip_backend* be) {
@@ -871,6 +881,10 @@ void qhip_backend_free_scratch(qhip_backend* be) {
   be->act = nullptr;
   be->act_cap = 0;
   memo_clear(be);
+  if (be->pact) (void)hipFree(be->pact);
+  be->placed -= be->pact_cap;
+  be->pact = nullptr;
+  be->pact_cap = 0;
   if (be->skwork) (void)hipFree(be->skwork);
   be->placed -= be->skwork_cap;
   be->skwork = nullptr;
@@ -1020,7 +1034,7 @@ const char* qhip_backend_describe(qhip_backend* be) {
   for (const auto& c : be->arena) weights += c.used;
   for (const auto& c : be->img_arena) gemv_img += c.used;
   for (const auto& kv : be->images) mmq_img += kv.second.bytes;
-  const size_t scratch = be->act_cap + be->skwork_cap;
+  const size_t scratch = be->act_cap + be->pact_cap + be->skwork_cap;
   char budget[48] = "no cap";
   if (be->budget) snprintf(budget, sizeof budget, "%zu MiB", be->budget >> 20);
   snprintf(be->desc, sizeof be->desc,

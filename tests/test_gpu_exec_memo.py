@@ -183,3 +183,54 @@ def test_decode_step_in_hip_graph(gpu, oracle, weights):
     finally:
         torch.cuda.synchronize()
         be.close()
+
+
+@pytest.mark.parametrize("captured", [False, True])
+def test_memo_mixed_prompt_quantizes_each_family_once(gpu, oracle, captured):
+    """Q4_K and Q6_K products of one prompt: the one reads Q8_K rows, the other
+    the activation image, and neither evicts the other's quantization."""
+    rows, cols, tokens = 300, 1024, 200
+    w = {tt: synth.make_weight(tt, rows, cols, seed=38, tag=tt) for tt in (po.TT_Q6_K, po.TT_Q4_K)}
+    x = synth.make_act(cols, tokens, seed=39)
+    be = ops.Backend(0)
+    try:
+        base = be.mem_placed()
+        be.set_act_memo(True)
+        lins = {tt: be.load_linear(tt, rows, cols, v) for tt, v in w.items()}
+        assert all(be.prepare_linear(lin) == 0 for lin in lins.values())
+        loaded = be.mem_placed()
+        assert be.lib.qhip_backend_alloc_scratch_k(be._h, cols, tokens) == 0
+        xd = torch.from_numpy(x).to(gpu)
+        outs = [(tt, torch.zeros((tokens, rows), device=gpu)) for tt in list(w) * 2]
+
+        def layer():
+            be.step_begin(0)
+            for tt, out in outs:
+                be.matvec_batch_k(out, lins[tt], xd, tokens)
+
+        if captured:
+            side = torch.cuda.Stream()
+            be.set_stream(side)
+            g = torch.cuda.CUDAGraph()
+            torch.cuda.synchronize()
+            with torch.cuda.graph(g, stream=side):
+                layer()
+        else:
+            layer()
+        assert be.act_stats() == (2, 2)
+        for i in range(2):
+            if captured:
+                x = synth.make_act(cols, tokens, seed=40 + i)
+                xd.copy_(torch.from_numpy(x))
+                g.replay()
+            torch.cuda.synchronize()
+            for tt, out in outs:
+                assert rel_l2(out.cpu().numpy(), oracle.matvec(tt, w[tt], x)) < TOL
+        be.set_stream(torch.cuda.current_stream())
+        if captured:
+            del g
+        be.lib.qhip_backend_free_scratch(be._h)
+        assert be.mem_placed() == loaded > base
+    finally:
+        torch.cuda.synchronize()
+        be.close()
