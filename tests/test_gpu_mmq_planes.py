@@ -60,9 +60,11 @@ def test_planes_match_oracle(gpu, oracle, backend, tt):
 
 # 17408 x 256 rows and K of one super-block: whole rounds of tiles and nothing
 # to slice; 66 x 8192: a few tiles, sliced; 4224 x 2048: a full round of
-# 128-token tiles of 256 rows and a sliced remainder
+# 128-token tiles of 256 rows and a sliced remainder; 700 x 1024 and x 2304: 18
+# whole tiles and 36 pieces of sliced ones, no multiples of the eight XCDs
 @pytest.mark.parametrize("tt", [po.TT_Q6_K, po.TT_Q3_K, po.TT_Q5_K])
-@pytest.mark.parametrize("rows,cols,tokens", [(17408, 256, 90), (66, 8192, 257), (4224, 2048, 2100)])
+@pytest.mark.parametrize("rows,cols,tokens", [(17408, 256, 90), (66, 8192, 257), (4224, 2048, 2100),
+                                              (700, 1024, 150), (700, 2304, 150)])
 def test_planes_grids(gpu, oracle, backend, tt, rows, cols, tokens):
     w = synth.make_weight(tt, rows, cols, seed=43, tag=tt)
     x = synth.make_act(cols, tokens, seed=44)
