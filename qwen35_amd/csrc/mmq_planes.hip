@@ -268,8 +268,9 @@ hipError_t launch_planes_prepare(int ttype, const void* w, long row_bytes, int r
 }
 
 // ---- the product -------------------------------------------------------------------------
-// Tiles of 128 rows x TK = 32 NA tokens.  Within a workgroup of four waves,
-// wave w takes row group w and all TK tokens, 16 at a time.  A super-block's 16
+// Tiles of 32 NW rows x TK = 32 NA tokens: 128 x 64 (four waves, two workgroups
+// per CU) or 256 x 128 (eight waves, one per CU; planes_plan).  Wave w takes row
+// group w and all TK tokens, 16 at a time.  A super-block's 16
 // plane fragments stay in registers; each activation fragment read from LDS
 // (16 tokens x 64 values) feeds four v_mfma_i32_16x16x64_i8 (two row halves,
 // two planes), isum = 64 C_hi + C_lo: the reference's per-super-block integer
@@ -284,15 +285,15 @@ hipError_t launch_planes_prepare(int ttype, const void* w, long row_bytes, int r
 // meanwhile.
 //
 // Grid: workgroups [0, nwhole) take whole tiles, as many full rounds of
-// resident workgroups (two per CU) as there are; the remaining tiles come last
+// resident workgroups as there are; the remaining tiles come last
 // and are cut into P slices over K, so that they fill the final, partial round.
 // P minimises the work of the busiest workgroup (at least four super-blocks a
 // slice).  Within each part a block's tile is XCD-contiguous (block b is
 // dispatched to XCD b % 8): the token tiles of one row tile, which share the
 // weights, run side by side on one XCD; the slices are ordered (group of ntt
 // tiles, slice, tile) for the same reason.  Blocks are dispatched as others
-// finish: the tiles of one round take 60-90 us each at [16384, 5120] x 2048
-// (contention, not work), and a persistent grid with a fixed share per
+// finish: the 256 x 128 tiles of one round take 60-90 us each at [16384, 5120]
+// x 2048 (contention, not work), and a persistent grid with a fixed share per
 // workgroup, though it saves each tile's prologue, was no faster than one
 // block per tile (387-411 against 372 us).  A sliced tile is finished
 // deterministically: each slice writes its partial tile to the workspace, the
@@ -578,22 +579,28 @@ __global__ __launch_bounds__(64 * NW, 2) void k_mmq_planes(const uint8_t* __rest
       }
 }
 
-static int planes_na(int tokens) { return tokens <= 256 ? 2 : 4; }
-static int planes_nw(int tokens) { return planes_na(tokens) == 2 ? 4 : 8; }
-
-// split = false: no tile is cut over K (no workspace needed)
-static PlPlan planes_plan(int rows, int cols, int tokens, bool split) {
-  PlPlan p{};
-  const int tk = 32 * planes_na(tokens);
+// A launch with tiles of 32 NA tokens (and 64 NA rows, 2 NA waves).  split =
+// false: no tile is cut over K (no workspace needed).
+struct PlLaunch {
+  PlPlan p;
+  int na;
+  long steps;  // super-blocks of the busiest workgroup slot
+};
+static PlLaunch planes_shape(int rows, int cols, int tokens, bool split, int na) {
+  PlLaunch l{};
+  PlPlan& p = l.p;
+  const int tk = 32 * na, nw = 2 * na;
+  l.na = na;
   p.nsb = cols / 256;
   p.ntt = (tokens + tk - 1) / tk;
-  const int nw = planes_nw(tokens), ntiles = p.ntt * ((rows + 32 * nw - 1) / (32 * nw));
+  const int ntiles = p.ntt * ((rows + 32 * nw - 1) / (32 * nw));
   const int cus = qhip_gpu_cu_count();
-  const int slots = 8 / nw * (cus > 0 ? cus : 256);  // resident workgroups: two per CU
+  const int slots = 8 / nw * (cus > 0 ? cus : 256);  // resident workgroups: eight waves per CU
   p.nwhole = ntiles / slots * slots;
   p.sk_tiles = ntiles - p.nwhole;
   p.P = 1;
   p.gw = 1;
+  l.steps = (long)(p.nwhole / slots + (p.sk_tiles > 0)) * p.nsb;
   if (p.sk_tiles > 0 && split && p.sk_tiles <= kSkMaxTiles) {
     // the slice count with the least work on the busiest workgroup (ties:
     // fewer slices), at least four super-blocks a slice; a slice costs its
@@ -608,22 +615,39 @@ static PlPlan planes_plan(int rows, int cols, int tokens, bool split) {
         p.P = q;
       }
     }
+    l.steps = (long)(p.nwhole / slots) * p.nsb + best;
     p.gw = p.ntt < p.sk_tiles ? p.ntt : p.sk_tiles;
   }
   if (p.P == 1) {  // nothing is sliced
     p.nwhole = ntiles;
     p.sk_tiles = 0;
   }
-  return p;
+  return l;
+}
+
+// Tiles of 128 x 64 up to 256 tokens, else of 256 x 128.  The large tile's
+// workgroup has a CU to itself and does twice the work per CU of two of the
+// small ones in 1.5 to 1.7 times their time, so below 2^25 weights, whose grid
+// may not fill the CUs with it, it is taken where it saves a third of the
+// steps.  us, small / large: Q5_K [1024, 1024] x 300 15.1 / 23.6, [2560, 2560]
+// x 300 22.0 / 34.5, x 2048 50.8 / 49.8, [9728, 2560] x 300 33.7 / 38.8, x 700
+// 62.9 / 52.0, x 2048 160 / 136; [14336, 4096] x 300 69.8 / 76.7, x 512 101 /
+// 78, x 2048 338 / 268 (from 2^25 weights always the large one).
+static PlLaunch planes_plan(int rows, int cols, int tokens, bool split) {
+  if (tokens <= 256) return planes_shape(rows, cols, tokens, split, 2);
+  if ((long)rows * cols < (1L << 25) &&
+      3 * planes_shape(rows, cols, tokens, true, 4).steps >= 2 * planes_shape(rows, cols, tokens, true, 2).steps)
+    return planes_shape(rows, cols, tokens, split, 2);
+  return planes_shape(rows, cols, tokens, split, 4);
 }
 
 // Workspace of the plane-image MMQ: tile counters, then one partial tile per
 // piece (none when no tile is sliced).
 long planes_work_bytes(int rows, int cols, int tokens) {
   if (rows <= 0 || tokens <= 0 || cols <= 0 || cols % 256) return 0;
-  const PlPlan p = planes_plan(rows, cols, tokens, true);
-  if (p.P <= 1) return 0;
-  return kSkCountBytes + (long)p.sk_tiles * p.P * 32L * planes_nw(tokens) * 32 * planes_na(tokens) * 4;
+  const PlLaunch l = planes_plan(rows, cols, tokens, true);
+  if (l.p.P <= 1) return 0;
+  return kSkCountBytes + (long)l.p.sk_tiles * l.p.P * (64L * l.na) * (32 * l.na) * 4;
 }
 
 hipError_t launch_mmq_planes(int ttype, const void* img, const void* xa, float* out, int rows, int cols, int tokens,
@@ -633,14 +657,15 @@ hipError_t launch_mmq_planes(int ttype, const void* img, const void* xa, float* 
       (long)tokens * ((rows + 127) / 128) > 0x3FFFFFFFL)
     return hipErrorInvalidValue;
   const long need = planes_work_bytes(rows, cols, tokens);
-  const PlPlan p = planes_plan(rows, cols, tokens, need > 0 && work && work_bytes >= need);
+  const PlLaunch l = planes_plan(rows, cols, tokens, need > 0 && work && work_bytes >= need);
+  const PlPlan& p = l.p;
   unsigned* cnt = (unsigned*)work;
   float* part = work ? (float*)((uint8_t*)work + kSkCountBytes) : nullptr;
 #define QHIP_PLANES(NW, NA, PL, MINS)                                                                            \
   hipLaunchKernelGGL((k_mmq_planes<NW, NA, PL, MINS>), dim3((unsigned)(p.nwhole + p.sk_tiles * p.P)),            \
                      dim3(64 * NW), 0, s, (const uint8_t*)img, (const uint8_t*)xa, out, rows, tokens, p, part, cnt)
 #define QHIP_PLANES_SIZE(PL, MINS)              \
-  if (planes_na(tokens) == 2)                   \
+  if (l.na == 2)                                \
     QHIP_PLANES(4, 2, PL, MINS);                \
   else                                          \
     QHIP_PLANES(8, 4, PL, MINS)
