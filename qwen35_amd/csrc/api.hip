@@ -113,28 +113,42 @@ static bool mmq_supported(int ttype) {
 //   IQ3_XXS  130 / 512    67 / 118 vs 83 / 172    34 / 55  vs 62 / 92
 //   IQ3_S    130 / 512    69 / 118 vs 91 / 186    34 / 56  vs 68 / 105
 //
-// Below the thresholds the two-plane image's 2.06 bytes a weight cost more
-// than the tile MMQ's decode (IQ4_XS [17408, 5120] x 64 50 vs 39 us, Q2_K
-// [9728, 2560] x 64 19.1 vs 18.4); Q6_K up to 64 tokens reads its fragment
-// image.  Q4_K stays on its fragment image, a quarter of the bytes: 512 tokens
-// [17408, 5120] 125 us against 133 from its planes.
+// Below the thresholds the two-plane image's 2.02 to 2.16 bytes a weight cost
+// more than the tile MMQ's decode (IQ4_XS [17408, 5120] x 64 50 vs 39 us, Q2_K,
+// of one plane and 1.16 bytes, [9728, 2560] x 64 19.1 vs 18.4).  Q4_K stays on
+// its fragment image, a quarter of the bytes: 512 tokens [17408, 5120] 125 us
+// against 133 from its planes.
 //
-// Q5_K to 128 tokens and Q6_K to 96 on rows below 12288 stay on the fragment
+// Q5_K to 128 tokens and Q6_K to 96 (wd_image_preferred) read the fragment
 // image, a third of the bytes, whose few-token launch needs no hand-off (us,
 // fragments / planes: Q5_K x 65 [9728, 2560] 20.3 / 33.5, [5120, 17408] 48.3 /
 // 63.9, x 128 [17408, 5120] 61.7 / 71.7, [5120, 17408] 64.5 / 66.6, x 160 84.5 /
-// 75.6; Q6_K x 96 [9728, 2560] 26.3 / 31.7, [2560, 9728] 26.8 / 34.7, [17408,
-// 5120] 62.7 / 66.8, [5120, 17408] 66.5 / 60.3).
+// 75.6).  Other Q6_K products of 65 to 128 tokens multiply the Q8_K rows from
+// the same planes (mmq_image_preferred; us, rows / activation image: [1024,
+// 4096] x 65 18.5 / 19.9, [2560, 2560] 19.4 / 20.4, [14336, 4096] 43.4 / 45.2,
+// [5120, 5120] x 97 29.9 / 31.3; at 160 the two meet, [5120, 5120] x 256 42.8 /
+// 33.0).
 bool wd_image_preferred(const GemvArgs& g);
+static int cus() {
+  const int n = qhip_gpu_cu_count();
+  return n > 0 ? n : 256;
+}
 bool planes_preferred(const GemvArgs& g) {
   if (g.tokens > 65535 || planes_image_bytes(g.ttype, g.rows, g.cols) <= 0 || !fast_ok(g)) return false;
   switch (g.ttype) {
-    case TT_Q6_K: case TT_Q5_K: return g.tokens > 64 && !wd_image_preferred(g);
+    case TT_Q6_K: return g.tokens > 128;
+    case TT_Q5_K: return g.tokens > 64 && !wd_image_preferred(g);
     case TT_Q2_K: return g.tokens > 64;
     case TT_Q3_K: return g.tokens > 24;
     case TT_IQ4_XS: case TT_IQ3_XXS: case TT_IQ3_S: return g.tokens > 128;
     default: return false;
   }
+}
+// Prompts of Q6_K whose Q8_K rows are multiplied from the plane image: up to 128
+// tokens, and where there is no room for the activation image
+bool mmq_image_preferred(const GemvArgs& g) {
+  return g.ttype == TT_Q6_K && g.tokens > 64 && mmq_image_bytes(g.ttype, g.rows, g.cols) > 0 && fast_ok(g) &&
+         !wd_image_preferred(g);
 }
 
 // Batches of a large Q6_K or Q4_K weight: the Exec mirror multiplies them
@@ -166,14 +180,26 @@ bool planes_preferred(const GemvArgs& g) {
 // = 3584 ([1024, 3584]: 16 workgroups walking four super-chunks) the image
 // loses to the GEMV up to 24 tokens (13.3 against 16.9 us there), so wider
 // Q8_0 rows keep the GGUF-row paths.
+//
+// Past 64 tokens (three and four 32-token tiles, whose weight reads meet in L2)
+// against the launches of planes_preferred: Q5_K to 128; Q6_K to 96 where all three tiles'
+// workgroups run at once ([2560, 12032] x 80 30.2 us / 36.1 from the planes and
+// the rows; [4096, 9728] 1.06 of it, [3584, 10240] 1.10) or the weight is not
+// too large ([5120, 8192] 34.5 / 37.3, [12288, 5120] 46.4 / 49.2, [16384, 2048]
+// 28.8 / 32.2; [10240, 8192] 59.9 / 57.0, [16384, 5120] 1.05, [24576, 2048]
+// 1.10, [16384, 1024] 1.08).
+static bool wd_q6k_three_tiles(const GemvArgs& g) {
+  if (3L * ((g.rows + 31) / 32) <= cus()) return g.cols < 12288;
+  return g.cols <= 8192 && (long)g.rows * g.cols < (1L << 26) && g.rows <= (g.cols < 2048 ? 12288 : 20480);
+}
 bool wd_image_preferred(const GemvArgs& g) {
   if (g.ttype == TT_Q8_0)
     return g.tokens >= 6 && g.cols <= 1024 && wd_image_bytes(g.ttype, g.rows, g.cols) > 0 && fast_ok(g);
   if (g.tokens < 2 || (long)g.rows * g.cols < (1L << 23) || !fast_ok(g)) return false;
-  const int most = g.ttype == TT_Q5_K ? 128 : g.ttype == TT_Q6_K ? (g.cols < 12288 ? 96 : 64) : 0x7FFFFFFF;
-  if (g.tokens > most || wd_image_bytes(g.ttype, g.rows, g.cols) <= 0) return false;
-  if (g.ttype == TT_Q6_K || g.ttype == TT_Q5_K) return true;
-  return g.ttype == TT_Q4_K && wd_image_bytes(g.ttype, g.rows, g.cols) > 0;
+  if (wd_image_bytes(g.ttype, g.rows, g.cols) <= 0) return false;
+  if (g.ttype == TT_Q5_K) return g.tokens <= 128;
+  if (g.ttype == TT_Q6_K) return g.tokens <= 64 || (g.tokens <= 96 && wd_q6k_three_tiles(g));
+  return g.ttype == TT_Q4_K;
 }
 
 // `work` (nullable): the split-K workspace of the MMQ (mmq_work_bytes)

@@ -25,6 +25,7 @@ namespace qhip {
 hipError_t dispatch_mul_mat(const GemvArgs& g, int path, void* work, long work_bytes, hipStream_t s);
 long mul_mat_work_bytes(const GemvArgs& g);
 bool planes_preferred(const GemvArgs& g);
+bool mmq_image_preferred(const GemvArgs& g);
 bool wd_image_preferred(const GemvArgs& g);
 }
 
@@ -636,6 +637,14 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
       return report("matvec", launch_mmq_wd_image(GemvArgs{ttype, img, be->act, out, rows, cols, k, row_bytes,
                                                            qhip_act_row_bytes(ttype, cols)}, work, work_bytes,
                                                   be->stream, true));
+  }
+  if (mmq_image_preferred(g)) {
+    // a prompt of a Q6_K weight on its Q8_K rows: the MMQ from its plane image
+    void* img = image_for(be, wdev, ttype, rows, cols, kImgMmq, &e);
+    if (e != hipSuccess) return report("MMQ image", e);
+    if (img)
+      return report("matvec", (hipError_t)qhip_launch_mul_mat_image(img, be->act, out, rows, cols, k, ttype, 0, 0,
+                                                                     work, work_bytes, be->stream));
   }
   return report("matvec", dispatch_mul_mat(g, QHIP_PATH_AUTO, work, work_bytes, be->stream));
 }

@@ -16,9 +16,10 @@ from test_gpu_mmq import rel_l2, to_dev, unit_scale_act, unit_scale_weight
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-5
-# format: the token count the route starts at
 STARTS = {po.TT_Q6_K: 65, po.TT_Q5_K: 65, po.TT_Q2_K: 65, po.TT_Q3_K: 25, po.TT_IQ4_XS: 129, po.TT_IQ3_XXS: 129,
           po.TT_IQ3_S: 129}
+FORMATS = [po.TT_Q6_K, po.TT_Q5_K, po.TT_Q2_K, po.TT_Q3_K, po.TT_IQ4_XS, po.TT_IQ3_XXS, po.TT_IQ3_S]
+START = 129
 
 
 @pytest.fixture
@@ -40,30 +41,29 @@ def product(be, tt, wd, rows, cols, x, images=True):
     return out, placed - be.mem_placed()
 
 
-@pytest.mark.parametrize("tt", list(STARTS))
+@pytest.mark.parametrize("tt", FORMATS)
 def test_planes_match_oracle(gpu, oracle, backend, tt):
     rows, cols = 333, 2048
     w = synth.make_weight(tt, rows, cols, seed=41, tag=tt)
     wd = to_dev(w, gpu)
-    for tokens in (STARTS[tt] - 1, STARTS[tt], 130, 256, 257, 300):
+    for tokens in (24, 25, 64, 65, START - 1, START, 130, 256, 257, 300):
         x = synth.make_act(cols, tokens, seed=42, tag=tokens)
         xd = to_dev(x, gpu)
         got, image = product(backend, tt, wd, rows, cols, xd)
         assert rel_l2(got.cpu().numpy(), oracle.matvec(tt, w, x)) < TOL
-        if tt != po.TT_Q6_K:  # which has a fragment image too
-            assert (image > 0) == (tokens >= STARTS[tt])
+        assert (image > 0) == (tokens >= STARTS[tt])
         again, _ = product(backend, tt, wd, rows, cols, xd)
         assert torch.equal(got, again)  # the slices are added in a fixed order
         plain, image = product(backend, tt, wd, rows, cols, xd, images=False)
         assert image == 0 and rel_l2(plain.cpu().numpy(), got.cpu().numpy()) < 1e-6
 
 
-# 17408 x 256 rows and K of one super-block: whole rounds of tiles and nothing
-# to slice; 66 x 8192: a few tiles, sliced; 4224 x 2048: a full round of
+# 17408 x 256 rows and K of one super-block: more than a round of whole tiles and
+# nothing to slice; 66 x 8192: a few tiles, sliced; 4224 x 2048: a full round of
 # 128-token tiles of 256 rows and a sliced remainder; 700 x 1024 and x 2304: 18
 # whole tiles and 36 pieces of sliced ones, no multiples of the eight XCDs
 @pytest.mark.parametrize("tt", [po.TT_Q6_K, po.TT_Q3_K, po.TT_Q5_K])
-@pytest.mark.parametrize("rows,cols,tokens", [(17408, 256, 90), (66, 8192, 257), (4224, 2048, 2100),
+@pytest.mark.parametrize("rows,cols,tokens", [(17408, 256, 250), (66, 8192, 257), (4224, 2048, 2100),
                                               (700, 1024, 150), (700, 2304, 150)])
 def test_planes_grids(gpu, oracle, backend, tt, rows, cols, tokens):
     w = synth.make_weight(tt, rows, cols, seed=43, tag=tt)
@@ -81,15 +81,18 @@ def test_planes_grids(gpu, oracle, backend, tt, rows, cols, tokens):
 @pytest.mark.parametrize("tt", [po.TT_Q6_K, po.TT_Q5_K, po.TT_Q3_K, po.TT_Q2_K, po.TT_IQ4_XS])
 @pytest.mark.parametrize("tokens", [140, 270])
 def test_planes_integers_exact(gpu, oracle, backend, tt, tokens):
-    """d = dmin = 1 and activations of Q8_K scale 1: every output is the exact
-    integer sum of its row (one super-block, below 2^24)."""
-    rows, cols = 70, 256
+    """d = dmin = 1 in one super-block of a row and 0 in the others, activations
+    of Q8_K scale 1: every output is that block's exact integer (below 2^24)."""
+    rows, cols = 70, 2048
     w = unit_scale_weight(tt, rows, cols, seed=45)
+    blk = w.reshape(rows, 8, -1)
+    at = {po.TT_Q6_K: 208, po.TT_Q3_K: 108, po.TT_Q2_K: 80}.get(tt, 0)
+    blk[:, np.arange(8) != 5, at:at + (4 if tt in (po.TT_Q5_K, po.TT_Q2_K) else 2)] = 0
     x = unit_scale_act(cols, tokens, seed=46)
     want = oracle.matvec(tt, w, x)
     assert np.abs(want).max() < 2 ** 24 and np.array_equal(want, np.rint(want))
-    got, _ = product(backend, tt, to_dev(w, gpu), rows, cols, to_dev(x, gpu))
-    assert np.array_equal(got.cpu().numpy(), want)
+    got, image = product(backend, tt, to_dev(w, gpu), rows, cols, to_dev(x, gpu))
+    assert image > 0 and np.array_equal(got.cpu().numpy(), want)
 
 
 def test_planes_largest_values(gpu, oracle, backend):
@@ -103,8 +106,8 @@ def test_planes_largest_values(gpu, oracle, backend):
     w6[:, 192:208] = 0x80
     w6[:, 208:210] = np.array([1.0], np.float16).view(np.uint8)
     for tt, w in ((po.TT_Q3_K, w3), (po.TT_Q6_K, w6)):
-        got, _ = product(backend, tt, to_dev(w, gpu), rows, cols, to_dev(x, gpu))
-        assert np.array_equal(got.cpu().numpy(), oracle.matvec(tt, w, x))
+        got, image = product(backend, tt, to_dev(w, gpu), rows, cols, to_dev(x, gpu))
+        assert image > 0 and np.array_equal(got.cpu().numpy(), oracle.matvec(tt, w, x))
 
 
 @pytest.mark.parametrize("shift", [0, 1])  # x 16-byte aligned, and 4 bytes past it
@@ -138,7 +141,7 @@ def test_activation_image_bytes(gpu, oracle, shift):
 
 def test_planes_captured_and_memo(gpu, oracle, backend):
     """A captured launch replays on new activations; with the memo on, a second
-    product of the same x reuses the image, and a a product of another activation
+    product of the same x reuses the image, and a product of another activation
     family does not meet it."""
     tt, rows, cols, tokens = po.TT_Q5_K, 300, 1024, 150
     w = synth.make_weight(tt, rows, cols, seed=48)
@@ -176,12 +179,14 @@ def test_planes_captured_and_memo(gpu, oracle, backend):
     assert (h1 - h0, m1 - m0) == (1, 2)
 
 
+@pytest.mark.parametrize("tt", [po.TT_Q3_K, po.TT_Q6_K])
 @pytest.mark.parametrize("room", [True, False])
-def test_planes_captured_after_reservation(gpu, oracle, backend, room):
+def test_planes_captured_after_reservation(gpu, oracle, backend, tt, room):
     """alloc_scratch_k and prepare_linear make a prompt capturable without an
     eager run before it, also at a token count that is no whole group of 32;
-    where the budget holds only the Q8_K rows, the product runs on those."""
-    tt, rows, cols, tokens = po.TT_Q3_K, 300, 1024, 37
+    where the budget holds only the Q8_K rows, the product runs on those (Q6_K
+    from the plane image still)."""
+    rows, cols, tokens = 300, 1024, 133
     w = synth.make_weight(tt, rows, cols, seed=51)
     wd = to_dev(w, gpu)
     lin = backend.wrap_linear(tt, rows, cols, wd)
@@ -190,7 +195,7 @@ def test_planes_captured_after_reservation(gpu, oracle, backend, room):
     if not room:
         backend.set_mem_budget(placed + cols // 256 * 292 * tokens + 256)
     assert backend.lib.qhip_backend_alloc_scratch_k(backend._h, cols, tokens) == 0
-    assert (backend.mem_placed() - placed >= cols // 256 * 292 * 64) == room
+    assert (backend.mem_placed() - placed >= cols // 256 * 292 * 160) == room
     x, out = torch.empty((tokens, cols), device=gpu), torch.empty((tokens, rows), device=gpu)
     side = torch.cuda.Stream()
     backend.set_stream(side)
@@ -205,3 +210,30 @@ def test_planes_captured_after_reservation(gpu, oracle, backend, room):
         torch.cuda.synchronize()
         assert rel_l2(out.cpu().numpy(), oracle.matvec(tt, w, xi)) < TOL
     backend.set_stream(torch.cuda.current_stream())
+    if tt == po.TT_Q6_K and not room:  # the bits of the public image product, unsplit as under the capture
+        rows_out = ops.mul_mat_image(tt, ops.mmq_image(tt, wd, rows, cols), ops.quantize_act(tt, x), rows, cols, tokens)
+        assert torch.equal(rows_out, out)
+
+
+def image_bytes(tt, rows, cols, planes):
+    group = {po.TT_Q6_K: (16512, 6720), po.TT_Q5_K: (17664, 5632), po.TT_Q3_K: (8320, 0), po.TT_Q2_K: (9472, 0),
+             po.TT_IQ4_XS: (16512, 0)}[tt]  # per 32 rows and 256 values: planes, fragments
+    return (rows + 31) // 32 * (cols // 256) * group[0 if planes else 1]
+
+
+# both sides of each line of the dispatch: tokens -> plane image, fragment image
+# or neither
+@pytest.mark.parametrize("tt,rows,cols,routes", [
+    (po.TT_Q6_K, 1640, 5120, {96: "frag", 97: "planes"}),
+    (po.TT_Q6_K, 2720, 8448, {96: "frag"}), (po.TT_Q6_K, 2752, 8448, {64: "frag", 65: "planes"}),
+    (po.TT_Q6_K, 16384, 1024, {65: "planes"}),
+])
+def test_prompt_routes(gpu, oracle, backend, tt, rows, cols, routes):
+    w = synth.make_weight(tt, rows, cols, seed=55, tag=rows).reshape(rows, -1)
+    wd = to_dev(w, gpu)
+    at = np.unique(np.r_[np.linspace(0, rows - 1, 40).astype(int), rows - 3:rows])
+    for tokens, route in routes.items():
+        x = synth.make_act(cols, tokens, seed=56)
+        got, image = product(backend, tt, wd, rows, cols, to_dev(x, gpu))
+        assert rel_l2(got.cpu().numpy()[:, at], oracle.matvec(tt, np.ascontiguousarray(w[at]), x)) < TOL
+        assert image == (0 if route is None else image_bytes(tt, rows, cols, route == "planes")), tokens
