@@ -119,6 +119,22 @@ static bool mmq_supported(int ttype) {
 // its fragment image, a quarter of the bytes: 512 tokens [17408, 5120] 125 us
 // against 133 from its planes.
 //
+// Up to 128 tokens on a small weight the tile MMQ cuts K over workgroups and the
+// planes' few tiles do not fill the CUs (us, planes / tile MMQ): Q5_K [2560,
+// 2560] x 65 21.3 / 15.0, [1024, 4096] 20.5 / 13.7 (from 2^23 weights it has the
+// fragment image); Q2_K [2048, 2048] x 65 15.9 / 13.1, [4096, 2304] 1.07 of it,
+// [2560, 5120] 0.91; Q3_K x 65 [2560, 2560] 16.7 / 15.3, [3072, 3072] 0.88, x 33
+// [2560, 6912] 1.04, [3584, 5120] 0.86, x 25 [2560, 9728] 0.93, [6144, 3584]
+// 1.02.  From 129 tokens the tile MMQ has no slices and the planes win at every
+// size, but for rows of fewer than eight super-blocks, which they do not cut
+// either: IQ4_XS there loses with fewer than 9/16 of a tile per CU ([4096, 1024]
+// x 200 1.14, x 257 0.96; [3072, 1024] x 300 1.10, x 384 0.92; [1024, 1024] x
+// 1024 1.05, x 2048 0.87), rows of 512 with fewer than two (8192 rows x 384
+// 1.08, x 512 0.97), the IQ3 formats a few percent less.  And three token tiles
+// of long rows in 9/8 to 3/2 tiles per CU: IQ4_XS [16384, 4096] x 160 60.8 /
+// 53.7, [14336, 4096] 57.5 / 53.1; [12288, 4096] 54.0 / 53.0, [17408, 5120] 71.4 /
+// 81.5, IQ3_S [16384, 4096] 60.9 / 60.1.
+//
 // Q5_K to 128 tokens and Q6_K to 96 (wd_image_preferred) read the fragment
 // image, a third of the bytes, whose few-token launch needs no hand-off (us,
 // fragments / planes: Q5_K x 65 [9728, 2560] 20.3 / 33.5, [5120, 17408] 48.3 /
@@ -129,18 +145,33 @@ static bool mmq_supported(int ttype) {
 // [5120, 5120] x 97 29.9 / 31.3; at 160 the two meet, [5120, 5120] x 256 42.8 /
 // 33.0).
 bool wd_image_preferred(const GemvArgs& g);
+static long tiles_of(const GemvArgs& g, int tile_rows) {  // of 64 tokens
+  return (long)((g.rows + tile_rows - 1) / tile_rows) * ((g.tokens + 63) / 64);
+}
 static int cus() {
   const int n = qhip_gpu_cu_count();
   return n > 0 ? n : 256;
 }
+// The tile MMQ (64 x 64 tiles, two workgroups per CU) in one full round: K
+// uncut and no CU idle.  Q5_K [16384, 2048] x 128 28.6 us against 30.1 from the
+// fragments and 33.1 from the planes, [16384, 1024] 18.5 / 20.3 / 19.7.
+static bool tile_mmq_full_round(const GemvArgs& g) { return tiles_of(g, 64) == 2L * cus(); }
 bool planes_preferred(const GemvArgs& g) {
   if (g.tokens > 65535 || planes_image_bytes(g.ttype, g.rows, g.cols) <= 0 || !fast_ok(g)) return false;
+  const long n = (long)g.rows * g.cols;
   switch (g.ttype) {
     case TT_Q6_K: return g.tokens > 128;
-    case TT_Q5_K: return g.tokens > 64 && !wd_image_preferred(g);
-    case TT_Q2_K: return g.tokens > 64;
-    case TT_Q3_K: return g.tokens > 24;
-    case TT_IQ4_XS: case TT_IQ3_XXS: case TT_IQ3_S: return g.tokens > 128;
+    case TT_Q5_K:
+      return g.tokens > 128 || (g.tokens > 64 && n >= (1L << 23) && !wd_image_preferred(g) && !tile_mmq_full_round(g));
+    case TT_Q2_K: return g.tokens > 128 || (g.tokens > 64 && n >= 3L << 22);
+    case TT_Q3_K:
+      return g.tokens > 128 || (g.tokens > 64 && n >= 1L << 23) || (g.tokens > 24 && n >= 17L << 20);
+    case TT_IQ4_XS: case TT_IQ3_XXS: case TT_IQ3_S: {
+      if (g.tokens <= 128) return false;
+      const long tiles = tiles_of(g, 128);
+      if (g.cols < 2048) return 16 * tiles >= (g.cols < 1024 ? 32L : 9L) * cus();
+      return g.ttype == TT_IQ3_S || g.tokens > 192 || g.cols < 4096 || 8 * tiles <= 9L * cus() || 2 * tiles > 3L * cus();
+    }
     default: return false;
   }
 }
@@ -182,7 +213,9 @@ bool mmq_image_preferred(const GemvArgs& g) {
 // Q8_0 rows keep the GGUF-row paths.
 //
 // Past 64 tokens (three and four 32-token tiles, whose weight reads meet in L2)
-// against the launches of planes_preferred: Q5_K to 128; Q6_K to 96 where all three tiles'
+// against the launches of planes_preferred: Q5_K to 128, but for rows of up to
+// eight super-blocks in more than 20480 ([32768, 1536] x 128 47.1 us / 37.1 from
+// the planes, [20480, 2048] 36.4 / 39.8); Q6_K to 96 where all three tiles'
 // workgroups run at once ([2560, 12032] x 80 30.2 us / 36.1 from the planes and
 // the rows; [4096, 9728] 1.06 of it, [3584, 10240] 1.10) or the weight is not
 // too large ([5120, 8192] 34.5 / 37.3, [12288, 5120] 46.4 / 49.2, [16384, 2048]
@@ -197,7 +230,8 @@ bool wd_image_preferred(const GemvArgs& g) {
     return g.tokens >= 6 && g.cols <= 1024 && wd_image_bytes(g.ttype, g.rows, g.cols) > 0 && fast_ok(g);
   if (g.tokens < 2 || (long)g.rows * g.cols < (1L << 23) || !fast_ok(g)) return false;
   if (wd_image_bytes(g.ttype, g.rows, g.cols) <= 0) return false;
-  if (g.ttype == TT_Q5_K) return g.tokens <= 128;
+  if (g.ttype == TT_Q5_K)
+    return g.tokens <= 96 || (g.tokens <= 128 && (g.cols > 2048 || (g.rows <= 20480 && !tile_mmq_full_round(g))));
   if (g.ttype == TT_Q6_K) return g.tokens <= 64 || (g.tokens <= 96 && wd_q6k_three_tiles(g));
   return g.ttype == TT_Q4_K;
 }

@@ -16,10 +16,8 @@ from test_gpu_mmq import rel_l2, to_dev, unit_scale_act, unit_scale_weight
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-5
-STARTS = {po.TT_Q6_K: 65, po.TT_Q5_K: 65, po.TT_Q2_K: 65, po.TT_Q3_K: 25, po.TT_IQ4_XS: 129, po.TT_IQ3_XXS: 129,
-          po.TT_IQ3_S: 129}
 FORMATS = [po.TT_Q6_K, po.TT_Q5_K, po.TT_Q2_K, po.TT_Q3_K, po.TT_IQ4_XS, po.TT_IQ3_XXS, po.TT_IQ3_S]
-START = 129
+START = 129  # the token count the route starts at on a small weight (Q6_K reads the plane image from 65)
 
 
 @pytest.fixture
@@ -46,12 +44,12 @@ def test_planes_match_oracle(gpu, oracle, backend, tt):
     rows, cols = 333, 2048
     w = synth.make_weight(tt, rows, cols, seed=41, tag=tt)
     wd = to_dev(w, gpu)
-    for tokens in (24, 25, 64, 65, START - 1, START, 130, 256, 257, 300):
+    for tokens in (64, 65, START - 1, START, 130, 256, 257, 300):
         x = synth.make_act(cols, tokens, seed=42, tag=tokens)
         xd = to_dev(x, gpu)
         got, image = product(backend, tt, wd, rows, cols, xd)
         assert rel_l2(got.cpu().numpy(), oracle.matvec(tt, w, x)) < TOL
-        assert (image > 0) == (tokens >= STARTS[tt])
+        assert (image > 0) == (tokens >= (65 if tt == po.TT_Q6_K else START))
         again, _ = product(backend, tt, wd, rows, cols, xd)
         assert torch.equal(got, again)  # the slices are added in a fixed order
         plain, image = product(backend, tt, wd, rows, cols, xd, images=False)
@@ -227,6 +225,17 @@ def image_bytes(tt, rows, cols, planes):
     (po.TT_Q6_K, 1640, 5120, {96: "frag", 97: "planes"}),
     (po.TT_Q6_K, 2720, 8448, {96: "frag"}), (po.TT_Q6_K, 2752, 8448, {64: "frag", 65: "planes"}),
     (po.TT_Q6_K, 16384, 1024, {65: "planes"}),
+    (po.TT_Q5_K, 1640, 5120, {128: "frag", 129: "planes"}),
+    # the tile MMQ in one full round | rows of few super-blocks in many rows
+    (po.TT_Q5_K, 16384, 1024, {96: "frag", 97: None, 128: None, 129: "planes"}),
+    (po.TT_Q5_K, 20512, 1024, {96: "frag", 97: "planes"}),
+    (po.TT_Q2_K, 2458, 5120, {64: None, 65: "planes"}), (po.TT_Q2_K, 2457, 5120, {128: None, 129: "planes"}),
+    (po.TT_Q3_K, 1639, 5120, {64: None, 65: "planes"}), (po.TT_Q3_K, 1638, 5120, {128: None, 129: "planes"}),
+    (po.TT_Q3_K, 3482, 5120, {24: None, 25: "planes"}), (po.TT_Q3_K, 3481, 5120, {64: None, 65: "planes"}),
+    # fewer than eight super-blocks a row: from 9/16 of a tile per CU, of 512 values two
+    (po.TT_IQ4_XS, 4096, 1024, {256: None, 257: "planes"}), (po.TT_IQ4_XS, 8192, 512, {448: None, 449: "planes"}),
+    # three token tiles of long rows: up to 9/8 tiles per CU, and past 3/2
+    (po.TT_IQ4_XS, 12288, 4096, {192: "planes"}), (po.TT_IQ4_XS, 12416, 4096, {128: None, 192: None, 193: "planes"}),
 ])
 def test_prompt_routes(gpu, oracle, backend, tt, rows, cols, routes):
     w = synth.make_weight(tt, rows, cols, seed=55, tag=rows).reshape(rows, -1)
