@@ -3055,18 +3055,27 @@ static hipError_t launch_mmq_rk_nw(const GemvArgs& g, hipStream_t s) {
 }
 
 // Waves of a workgroup: with at most one workgroup per CU the waves of a group
-// of rows are all the CU has, so eight, and twelve on long rows; past that four
-// (eight up to 16 tokens within two workgroups per CU), as the stages of more
-// waves keep workgroups off the CU.  Weights from HBM, quantize and product, us
-// with 4 / 8 / 12 waves: Q5_K [4096, 4096] x 64 16.0 / 12.7 / 13.1, [5120, 17408]
-// x 8 31.8 / 22.5 / 20.4, [9728, 2560] x 8 10.8 / 10.2 / 11.5 and x 64 17.5 /
-// 23.7 / 24.7; Q4_K [2560, 9728] x 8 18.5 / 12.7 / 12.3 (all four before);
-// Q6_K [17408, 5120] x 16 26.6 / 27.2 / 30.0 (all twelve before).
+// of rows are all the CU has, so eight, and twelve on long rows or where they
+// take fewer steps over K; past that four (eight up to 16 tokens within two
+// workgroups per CU, to 8 where four divide K and eight do not), as the stages
+// of more waves keep workgroups off the CU.  Weights
+// from HBM, quantize and product, us with 4 / 8 / 12 waves: Q5_K [4096, 4096] x
+// 64 16.0 / 12.7 / 13.1, [5120, 17408] x 8 31.8 / 22.5 / 20.4, [9728, 2560] x 8
+// 10.8 / 10.2 / 11.5 and x 64 17.5 / 23.7 / 24.7; Q4_K [2560, 9728] x 8 18.5 / 12.7
+// / 12.3, [12288, 3072] x 16 12.3 / 13.2 / 13.8; Q6_K [17408, 5120] x 16 26.6 /
+// 27.2 / 30.0, [5120, 5120] x 2 15.2 / 12.0 / 10.8, [8192, 2560] x 8 11.7 / 10.9 /
+// 9.7, [4096, 8192] x 8 21.2 / 15.1 / 15.6 and x 9 24.0 / 17.9 / 17.2 (Q4_K x 16
+// 18.8 / 13.8 / 14.1).
 static int rk_waves(const GemvArgs& g) {
-  const int cus0 = qhip_gpu_cu_count(), cus = cus0 > 0 ? cus0 : 256;
+  const int cus0 = qhip_gpu_cu_count(), cus = cus0 > 0 ? cus0 : 256, nsb = g.cols / 256;
   const long wgs = (long)((g.rows + 31) / 32) * ((g.tokens + 31) / 32);
-  if (wgs <= cus) return g.cols >= 9216 && g.tokens <= 32 ? 12 : 8;
-  return g.tokens <= 16 && wgs <= 2L * cus ? 8 : 4;
+  if (wgs <= cus) {
+    if (g.tokens <= 32 && nsb >= 36) return 12;
+    const bool fewer = (nsb + 11) / 12 < (nsb + 7) / 8 && (nsb <= 28 || (g.ttype == TT_Q6_K && g.tokens > 8));
+    return g.tokens <= 16 && fewer ? 12 : 8;
+  }
+  const int most = nsb <= 12 && nsb % 8 == 4 ? 8 : 16;
+  return wgs <= 2L * cus && g.tokens <= most ? 8 : 4;
 }
 
 // Whether the launch from the fragment image keeps K inside the workgroup: the

@@ -31,7 +31,8 @@ def product(tt, wd, rows, cols, x, images=True):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("tt", [po.TT_Q4_K, po.TT_Q5_K, po.TT_Q6_K])
-@pytest.mark.parametrize("rows,cols", [(8195, 1024), (6570, 1280), (1000, 9216)])
+@pytest.mark.parametrize("rows,cols", [(8195, 1024), (6570, 1280), (1000, 9216), (1640, 5120),
+                                       (11000, 1280)])
 def test_fragments_match_oracle(gpu, oracle, tt, rows, cols):
     w = synth.make_weight(tt, rows, cols, seed=61, tag=tt)
     wd = to_dev(w, gpu)
