@@ -1,12 +1,13 @@
 // mmq_planes.hip -- the prompt MMQ of the super-block formats from a weight's
-// plane image and an activation image (int8 MFMA, exact integers).
+// plane image and an activation image (int8 MFMA, exact integers); all of them
+// but Q4_K, whose prompts read its fragment image.
 //
 // Plane image.  Every value of a super-block format enters its block integer
 // as p = scale * value, an integer (Q6_K int8 scale x [-32, 31],
-// kernels256.c:200-212, :720-738; Q5_K / Q4_K 6 bits x 5 / 4 bits, :605-629,
-// :474-498; IQ4_XS 6 signed bits x codebook, iq_kernels.c:967-1001; IQ3_XXS /
-// IQ3_S odd scale x signed grid value, :612-643, :1728-1772; Q3_K 6 signed
-// bits x [-4, 3], kernels256.c:349-369; Q2_K 4 bits x 2 bits, :232-257).  The
+// kernels256.c:200-212, :720-738; Q5_K 6 bits x 5 bits, :605-629; IQ4_XS 6
+// signed bits x codebook, iq_kernels.c:967-1001; IQ3_XXS / IQ3_S odd scale x
+// signed grid value, :612-643, :1728-1772; Q3_K 6 signed bits x [-4, 3],
+// kernels256.c:349-369; Q2_K 4 bits x 2 bits, :232-257).  The
 // image holds p as one int8 plane where it fits (Q2_K at most 45; Q3_K as -p
 // in [-128, 124] with -d), else split exactly as p = 64 hi + lo (lo = p & 63,
 // hi = p >> 6: |p| < 2^13).  Per 32-row group and super-block: each plane's 8
@@ -35,7 +36,7 @@ typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
 // planes and mins of a format; image bytes per 32-row group and super-block
 constexpr int pl_planes(int tt) { return tt == TT_Q3_K || tt == TT_Q2_K ? 1 : 2; }
-constexpr bool pl_mins(int tt) { return tt == TT_Q4_K || tt == TT_Q5_K || tt == TT_Q2_K; }
+constexpr bool pl_mins(int tt) { return tt == TT_Q5_K || tt == TT_Q2_K; }
 constexpr int pl_grp(int planes, bool mins) { return 8192 * planes + 128 + (mins ? 128 + 1024 : 0); }
 constexpr int kActGrp = 9344;       // activation image bytes per 32-token group and super-block
 constexpr int kActSums = 8192, kActScale = 9216;
@@ -103,8 +104,8 @@ hipError_t launch_quantize_mmq_act(const float* x, void* out, int cols, int toke
 // ---- the plane image ---------------------------------------------------------------------
 bool planes_format(int ttype) {
   switch (ttype) {
-    case TT_Q6_K: case TT_Q5_K: case TT_Q4_K: case TT_Q3_K: case TT_Q2_K: case TT_IQ4_XS: case TT_IQ3_XXS:
-    case TT_IQ3_S: return true;
+    case TT_Q6_K: case TT_Q5_K: case TT_Q3_K: case TT_Q2_K: case TT_IQ4_XS: case TT_IQ3_XXS: case TT_IQ3_S:
+      return true;
     default: return false;
   }
 }
@@ -134,7 +135,7 @@ __device__ __forceinline__ int pl_scale(const uint8_t* blk, int e0) {
   const int s = e0 >> 5, g = e0 >> 4;
   int sc = 0, mn;
   if constexpr (TT == TT_Q6_K) sc = (int)(int8_t)blk[192 + g];
-  else if constexpr (TT == TT_Q4_K || TT == TT_Q5_K) pl_k_scale(blk + 4, s, sc, mn);
+  else if constexpr (TT == TT_Q5_K) pl_k_scale(blk + 4, s, sc, mn);
   else if constexpr (TT == TT_IQ4_XS)
     sc = (int)(((blk[4 + s / 2] >> (4 * (s % 2))) & 15u) | (((pl_ld16(blk + 2) >> (2 * s)) & 3u) << 4)) - 32;
   else if constexpr (TT == TT_IQ3_XXS) sc = 2 * (int)(pl_ld16(blk + 68 + 4 * s) >> 12) + 1;
@@ -159,11 +160,9 @@ __device__ __forceinline__ int pl_value(const uint8_t* blk, int e) {
     uint32_t lq = blk[64 * h + 32 * (q & 1) + l];
     lq = q >= 2 ? (lq >> 4) : (lq & 15u);
     return (int)(lq | (((blk[128 + 32 * h + l] >> (2 * q)) & 3u) << 4)) - 32;
-  } else if constexpr (TT == TT_Q4_K || TT == TT_Q5_K) {
-    const uint32_t b = blk[(TT == TT_Q5_K ? 48 : 16) + 32 * (s >> 1) + l];
-    int v = (int)((s & 1) ? (b >> 4) : (b & 15u));
-    if constexpr (TT == TT_Q5_K) v |= (int)((blk[16 + l] >> s) & 1u) << 4;
-    return v;
+  } else if constexpr (TT == TT_Q5_K) {
+    const uint32_t b = blk[48 + 32 * (s >> 1) + l];
+    return (int)((s & 1) ? (b >> 4) : (b & 15u)) | ((int)((blk[16 + l] >> s) & 1u) << 4);
   } else if constexpr (TT == TT_IQ4_XS) {
     const uint32_t b = blk[8 + 16 * s + (l & 15)];
     const uint32_t nib = l < 16 ? (b & 15u) : (b >> 4);
@@ -258,7 +257,7 @@ hipError_t launch_planes_prepare(int ttype, const void* w, long row_bytes, int r
   const dim3 grid((unsigned)((n + 255) / 256));
   return dispatch_type(ttype, [&](auto tt) {
     constexpr int TT = decltype(tt)::value;
-    if constexpr (act32(TT)) return hipErrorInvalidValue;
+    if constexpr (act32(TT) || TT == TT_Q4_K) return hipErrorInvalidValue;
     else {
       hipLaunchKernelGGL(k_planes_prepare<TT>, grid, dim3(256), 0, s, (const uint8_t*)w, (uint8_t*)img, rows, row_bytes,
                          cols / 256, n);
