@@ -410,12 +410,13 @@ void qhip_backend_free_linear(qhip_backend *be, qhip_linear *w);
  * 1.02x; built in load order, so adjacent weights get adjacent images and
  * matvecPair stays one launch), the fragment image of a Q6_K, Q5_K or Q4_K weight
  * with rows * cols >= 2^23 (qhip_launch_wd_prepare, the GGUF bytes once more;
- * matvec_batch_k reads it from 2 tokens, Q6_K up to 64, on rows below 12288 to
- * 96, Q5_K to 128) or of a Q8_0 weight with cols <= 1024 (from 6 tokens) and the
- * plane image of the other super-block formats' and Q6_K's prompts (Q6_K,
- * IQ4_XS and the IQ3 formats 2.02 bytes a weight, Q5_K 2.16, Q3_K 1.02, Q2_K
- * 1.16; read past the fragment image's tokens, from 65 where there is none, Q3_K
- * from 25, IQ4_XS and the IQ3 formats from 129).  A program that decodes only
+ * matvec_batch_k reads it from 2 tokens, Q6_K up to 64 or 96 and Q5_K to 96 or
+ * 128 by the weight's shape) or of a Q8_0 weight with cols <= 1024 (from 6
+ * tokens) and the plane image of the other super-block formats' and Q6_K's
+ * prompts (Q6_K, IQ4_XS and the IQ3 formats 2.02 bytes a weight, Q5_K 2.16, Q3_K
+ * 1.02, Q2_K 1.16; read from 129 tokens, Q6_K, Q5_K, Q3_K and Q2_K on larger
+ * weights also below that: Q6_K and Q5_K past the fragment image's tokens, Q2_K
+ * from 65, Q3_K from 25).  A program that decodes only
  * saves the MMQ images' time and room with qhip_backend_set_mmq_images(be, 0).
  * 0 = built or nothing to build; QHIP_DECLINE = not all built (images off, or
  * past the memory budget): the products then read the GGUF bytes.

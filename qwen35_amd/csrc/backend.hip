@@ -51,11 +51,12 @@ struct qhip_backend {
   // against the budget) until free_scratch or destroy.
   bool graph_seen = false;
   std::vector<std::pair<void*, size_t>> retired;
-  // MMQ images of Q6_K weights: the plane image of the prefill MMQ
-  // (qhip_launch_mmq_prepare, kind kImgMmq) and the fragment image of the
-  // few-token MMQ (qhip_launch_wd_prepare, kind kImgFrag), built by
-  // prepare_linear or by the first product that reads them outside a graph
-  // capture, kept until free_linear / destroy.  Keyed by the whole linear
+  // MMQ images of the super-block formats' and small Q8_0 weights: the plane
+  // image of a prompt (launch_planes_prepare, kind kImgMmq) and the fragment
+  // image of a few tokens (launch_wd_prepare, kind kImgFrag; Q4_K's also of a
+  // prompt), built by prepare_linear or by the first product that reads them
+  // outside a graph capture, kept until free_linear, destroy or until their
+  // room is needed (give_back_image).  Keyed by the whole linear
   // (device bytes, type, rows, cols) and the kind: a different weight wrapped
   // at a reused address never meets a stale image.
   struct ImageKey {
@@ -75,12 +76,13 @@ struct qhip_backend {
   };
   std::map<ImageKey, Image> images;
   bool images_on = true;
-  // GEMV images of the 32-value 4-bit formats (gemv_image.hip), keyed by the
-  // device address of the first GGUF row they mirror.  Their bytes come from
-  // a bump arena of their own, so images built in load order are adjacent
-  // exactly when their weights are, and an adjacent matvecPair stays one
-  // launch.  free_linear drops the entries over the weight's rows; the arena
-  // memory is returned at destroy, as the weights' is.
+  // GEMV images (IQ4_NL, Q4_0, Q8_0 and the K-quants but Q4_K;
+  // gemv_image.hip), keyed by the device address of the first GGUF row they
+  // mirror.  Their bytes come from a bump arena of their own, so images built
+  // in load order are adjacent when their weights are, and an adjacent
+  // matvecPair stays one launch.  free_linear drops the entries over the
+  // weight's rows; the arena memory is returned at destroy, as the weights'
+  // is, or when its room is needed (give_back_image).
   struct GImage {
     uint8_t* img;
     int ttype, rows, cols;

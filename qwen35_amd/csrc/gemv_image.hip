@@ -352,13 +352,14 @@ bool gemv_image_preferred(const GemvArgs& g) {
          (!gemv_fused_preferred(g) || (long)g.rows * g.cols >= (1L << 25) || !gemv_fused_one_round(g));
 }
 
-// ---- K-quant GEMV image (Q4_K, Q6_K) --------------------------------------------
-// The layout is KImg's (qhip_device.hpp): the GGUF row's bytes with each
+// ---- K-quant GEMV images ---------------------------------------------------------
+// Q2_K, Q3_K and Q5_K: ImgUnit's layout, each unit's own bits (qhip_device.hpp).
+// Q4_K and Q6_K: the layout is KImg's (qhip_device.hpp): the GGUF row's bytes with each
 // unit's 16-byte pieces grouped by piece over chunks of 64 units, so that the
 // lanes of a wave, taking consecutive units, load one contiguous span per
 // instruction; the headers (Q4_K) or scales and d (Q6_K) after the pieces.
-// The GEMV, fused and split-K launchers of gemv.hip read it when g.kimg, with
-// the activation in the reference Q8_K layout.
+// The GEMV launchers of gemv.hip (for Q4_K and Q6_K the fused and split-K ones
+// too) read them when g.kimg, with the activation in the reference Q8_K layout.
 bool gemv_kimage_format(int ttype) { return kimage_format(ttype); }
 bool gemv_kimage_own(int ttype) { return kimage_own(ttype); }
 long gemv_image_row_bytes(int ttype, int cols, long row_bytes) { return kimage_row_bytes(ttype, cols, row_bytes); }

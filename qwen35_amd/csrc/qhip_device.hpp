@@ -218,11 +218,11 @@ __device__ __forceinline__ uint32_t quant_q8_K_lane(const float* v, int& gsum, f
 }
 
 // ---- wave reductions --------------------------------------------------------------
-// Sum of v over the 64 lanes of a wave, in lane 63, by DPP.  Adjacent lanes and lane pairs within quads (quad_perm), then the mirrored
-// half-rows and rows give every lane of a 16-lane row the row's sum;
-// row_bcast:15 adds row 0's sum into row 1 and row 2's into row 3,
-// row_bcast:31 then adds rows 0 + 1 into rows 2 and 3.  The order of the
-// additions is fixed, so the result is deterministic.
+// Sum of v over the 64 lanes of a wave, in lane 63, by DPP.  Adjacent lanes and
+// lane pairs within quads (quad_perm), then the mirrored half-rows and rows give
+// every lane of a 16-lane row the row's sum; row_bcast:15 adds row 0's sum into
+// row 1 and row 2's into row 3, row_bcast:31 then adds rows 0 + 1 into rows 2
+// and 3.  The order of the additions is fixed, so the result is deterministic.
 __device__ __forceinline__ float wave_sum_to_lane63(float v) {
   v += dpp_f32<0xB1>(v);         // quad_perm [1, 0, 3, 2]
   v += dpp_f32<0x4E>(v);         // quad_perm [2, 3, 0, 1]

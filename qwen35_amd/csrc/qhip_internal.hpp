@@ -83,7 +83,7 @@ hipError_t launch_mmq_prepare(int ttype, const void* w, long row_bytes, int rows
 // (the plane image) has one shape and ignores bt, br
 hipError_t launch_mmq_image(const GemvArgs& g, int bt, int br, void* work, long work_bytes, hipStream_t s);
 // Plane image and activation image of the prompt MMQ (mmq_planes.hip): the
-// super-block formats, whose block integers are sums of scale * value.  The
+// super-block formats but Q4_K, whose block integers are sums of scale * value.  The
 // workspace: planes_work_bytes (0: none needed), its first kSkCountBytes zero;
 // without it no tile is cut over K.
 bool planes_format(int ttype);
