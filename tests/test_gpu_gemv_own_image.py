@@ -77,26 +77,41 @@ def test_q3_image_on_short_rows(gpu, oracle, backend):
         assert rel_l2(got, plain) < 1e-6
 
 
+# 250 rows: the images' bytes are no multiple of the arena's alignment, so two
+# adjacent weights' images are not adjacent, and the pair gets an image of its own
+@pytest.mark.parametrize("rows", [256, 250])
 @pytest.mark.parametrize("tt", FORMATS)
-def test_own_image_pair_and_capture(gpu, oracle, backend, tt):
+def test_own_image_pair_and_capture(gpu, oracle, backend, tt, rows):
     """Adjacent weights with adjacent images, in one launch; captured and
     replayed on new activations; and one weight of the pair alone."""
-    rows, cols = 256, 5120
+    cols = 5120
     w = synth.make_weight(tt, 2 * rows, cols, seed=55, tag=tt)
     wd = torch.from_numpy(w).to(gpu)
     half = wd.numel() // 2
     a = backend.wrap_linear(tt, rows, cols, wd.view(-1)[:half])
     b = backend.wrap_linear(tt, rows, cols, wd.view(-1)[half:])
+    assert backend.lib.qhip_backend_alloc_scratch(backend._h, cols) == 0
+    backend.set_mmq_images(False)  # the GEMV images alone
+    before = backend.mem_placed()
     backend.prepare_linear(a)
     backend.prepare_linear(b)
     xd = torch.from_numpy(synth.make_act(cols, 1, seed=56, tag=0)).to(gpu)
     pair = torch.empty(2 * rows, device=gpu)
     placed = backend.mem_placed()
+    row_bytes = {po.TT_Q2_K: 84, po.TT_Q3_K: 114, po.TT_Q5_K: 180}[tt] * (cols // 256)
+    image = (row_bytes + 15) // 16 * 16 * rows
+    adjacent = image % 256 == 0
+    assert adjacent == (rows == 256)
+    assert placed - before == 2 * ((image + 255) // 256 * 256)
     backend.matvec_pair(pair, a, b, xd[0])
+    # in one launch from both images, or from one built for the pair
+    assert backend.mem_placed() - placed == (0 if adjacent else (2 * image + 255) // 256 * 256)
+    placed = backend.mem_placed()
     want = oracle.matvec(tt, w, xd.cpu().numpy())[0]
     assert rel_l2(pair.cpu().numpy(), want) < 1e-5
     second = matvec(backend, b, xd, rows)
     assert rel_l2(second[0], want[rows:]) < 1e-5
+    assert np.array_equal(second[0], pair.cpu().numpy()[rows:])
     stream = torch.cuda.Stream()
     backend.set_stream(stream)
     out = torch.empty(1, rows, device=gpu)
@@ -110,7 +125,7 @@ def test_own_image_pair_and_capture(gpu, oracle, backend, tt):
         graph.replay()
         torch.cuda.synchronize()
         assert rel_l2(out.cpu().numpy()[0], oracle.matvec(tt, w, x)[0][:rows]) < 1e-5
-    assert backend.mem_placed() >= placed
+    assert backend.mem_placed() == placed  # the captured launch, too, read an image that was there
 
 
 @pytest.mark.parametrize("tt", FORMATS)
