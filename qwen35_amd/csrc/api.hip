@@ -469,6 +469,13 @@ int qhip_launch_mul_mat_vec_q8_0(const void* d_w, const void* d_xq, float* d_out
 
 int qhip_launch_quantize_mul_mat_vec(const void* d_w, const float* d_x, void* d_xq_out, float* d_out,
                                      int rows, int cols, int ttype, void* stream) {
+  return quantize_mul_mat_vec(d_w, d_x, d_xq_out, d_out, rows, cols, ttype, 0, S(stream));
+}
+
+}  // extern "C"
+
+int qhip::quantize_mul_mat_vec(const void* d_w, const float* d_x, void* d_xq_out, float* d_out, int rows, int cols,
+                               int ttype, int layout, hipStream_t s) {
   GemvArgs g;
   hipError_t e = make_args(d_w, d_x, d_out, rows, cols, 1, ttype, g);
   if (e != hipSuccess) return (int)e;
@@ -476,8 +483,10 @@ int qhip_launch_quantize_mul_mat_vec(const void* d_w, const float* d_x, void* d_
   if (rows == 0) return 0;
   // float4 activation reads: x 16-byte aligned
   if (!fast_ok(g) || ((uintptr_t)d_x & 15u) || !gemv_fused_fits(ttype, cols)) return QHIP_DECLINE;
-  return (int)launch_gemv_fused(g, d_x, d_xq_out, 0, 0, 0, S(stream));
+  return (int)launch_gemv_fused(g, d_x, d_xq_out, 0, 0, 0, s, layout);
 }
+
+extern "C" {
 
 int qhip_launch_quantize_mul_mat_vec_tuned(const void* d_w, const float* d_x, void* d_xq_out, float* d_out, int rows,
                                            int cols, int ttype, int lanes_per_row, int rows_per_lane,

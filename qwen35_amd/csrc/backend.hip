@@ -499,19 +499,18 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
   // the activation family: Q8_0 rows for 32-value weight blocks, Q8_K for
   // 256-value super-blocks (backend_cpu.zig:42-50 actFamily)
   const int fam = qhip_quant_act_block_elems(ttype);
+  const int sfam = kFamSplit + gemv_image_layout(ttype, cols);  // of this weight's GEMV image, if it has one
   if (k == 1 && be->gemv_images_on) {
     // IQ4_NL, Q4_0 and Q8_0 on larger matrices: split quantize + GEMV from the
     // weight's GEMV image.  The one-launch form is out where x is not aligned
-    // for it; with the memo on it would quantize once for this product only:
-    // the next one of x would read the GGUF rows.
+    // for it, or quantized already.
     const GemvArgs g1{ttype, wdev, x, out, rows, cols, 1, row_bytes, qhip_act_row_bytes(ttype, cols)};
-    const bool only = be->memo_on || ((uintptr_t)x & 15u);
+    const bool only = ((uintptr_t)x & 15u) || (be->memo_on && be->memo.holds(x, cols, 1, sfam));
     if ((only ? gemv_image_pays(g1) : gemv_image_preferred(g1)) && act_ready(be, act_bytes_for(cols, 1))) {
       hipError_t ei;
       uint8_t* img = gimage_for(be, wdev, ttype, rows, cols, row_bytes, &ei);
       if (ei != hipSuccess) return report("GEMV image", ei);
       if (img) {
-        const int sfam = kFamSplit + gemv_image_layout(ttype, cols);
         const bool hs = be->memo_on && be->memo.holds(x, cols, 1, sfam);
         if (be->memo_on) (hs ? be->memo_hits : be->memo_misses)++;
         if (!hs) {
@@ -582,6 +581,10 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
     const bool split = gemv_splitk_preferred(g1);
     if (split || gemv_fused_preferred(g1)) {
       void* xq_out = nullptr;
+      // a weight with a GEMV image leaves the activation in that image's
+      // layout: the next product of x is then the image's GEMV alone
+      const bool to_image = !split && be->memo_on && be->gemv_images_on && gemv_image_pays(g1) &&
+                            gimage_lookup(be, wdev, ttype, rows, cols, row_bytes);
       if (be->memo_on) {
         const hipError_t ea = ensure_act(be, act_bytes_for(cols, 1));
         if (ea != hipSuccess) return report("activation scratch", ea);
@@ -596,10 +599,10 @@ static int run(qhip_backend* be, float* out, const void* wdev, int ttype, int ro
         rc = qhip_launch_quantize_mul_mat_vec_split(wdev, x, xq_out, out, rows, cols, ttype, 0, 0, 0, be->skwork,
                                                     (long)be->skwork_cap, be->stream);
       } else {
-        rc = qhip_launch_quantize_mul_mat_vec(wdev, x, xq_out, out, rows, cols, ttype, be->stream);
+        rc = quantize_mul_mat_vec(wdev, x, xq_out, out, rows, cols, ttype, to_image ? sfam - kFamSplit : 0, be->stream);
       }
       if (rc != QHIP_DECLINE) {
-        if (rc == 0 && xq_out) be->memo = {x, cols, 1, fam};
+        if (rc == 0 && xq_out) be->memo = {x, cols, 1, to_image ? sfam : fam};
         return report("matvec", (hipError_t)rc);
       }
     }

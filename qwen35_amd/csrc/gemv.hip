@@ -274,7 +274,13 @@ __host__ __device__ constexpr long fused_lds_bytes(int ttype, int cols) {
 // cnt[tile]) adds the partials in slice order, writes y and puts the counter
 // back to zero, so the result does not depend on completion order.  No
 // workgroup waits for another: the last one to arrive does the sum.
-template <int TT, int NR, int WGS, bool SK = false>
+//
+// The quantized activation goes to XQ in the reference layout, or, SPLIT (not
+// SK), in the split layout of the GEMV image whose T and P slice_units and
+// slice_wbytes are (gemv_image.hip).  An instantiation of its own: the branch in
+// every launch took 0.9% of 24 layers of [3584, 1024] and [1024, 3584] (228.6 ->
+// 230.6 us).
+template <int TT, int NR, int WGS, bool SK = false, bool SPLIT = false>
 __global__ __launch_bounds__(WGS) void k_gemv_q(const uint8_t* __restrict__ W, const float* __restrict__ X,
                                                  uint8_t* __restrict__ XQ, float* __restrict__ Y, int rows,
                                                  int cols, long row_bytes, int upr, int team,
@@ -341,7 +347,11 @@ __global__ __launch_bounds__(WGS) void k_gemv_q(const uint8_t* __restrict__ W, c
     if (b < nblk) {
       *(uint32_t*)(qs + split_off(32 * b + qo)) = packed;
       if (qo == 0) dsc[b] = h2f(hb);
-      if (out_q) {
+      if (SPLIT && out_q) {
+        const int T = slice_units, P = (int)slice_wbytes, u = b >> 1, e = b & 1, p = u / T, j = u - p * T;
+        *(uint32_t*)(XQ + 16L * (((2 * p + e) * 2 + (qo >> 4)) * T + j) + (qo & 15)) = packed;
+        if (qo == 0) *(float*)(XQ + 64L * upr + 8L * (j * P + p) + 4 * e) = h2f(hb);
+      } else if (out_q) {
         uint8_t* ob = XQ + 34L * b;
         *(uint16_t*)(ob + 2 + qo) = (uint16_t)packed;
         *(uint16_t*)(ob + 4 + qo) = (uint16_t)(packed >> 16);
@@ -995,7 +1005,8 @@ static hipError_t launch_gemv_multiwave(const GemvArgs& g, int nr, int wv, hipSt
 }
 
 template <int TT, int NR, int WGS>
-static hipError_t launch_gemv_q_t(const GemvArgs& g, const float* x, void* xq_out, int team, hipStream_t s) {
+static hipError_t launch_gemv_q_t(const GemvArgs& g, const float* x, void* xq_out, int layout, int team,
+                                  hipStream_t s) {
   const int upr = g.cols / 64;
   if (team > 64) team = 64;
   const int tpw = 64 / team;
@@ -1003,23 +1014,32 @@ static hipError_t launch_gemv_q_t(const GemvArgs& g, const float* x, void* xq_ou
   const long waves = (teams + tpw - 1) / tpw;
   const unsigned grid = (unsigned)((waves + WGS / 64 - 1) / (WGS / 64));
   const size_t lds = (size_t)fused_lds_bytes(TT, g.cols);
-  hipLaunchKernelGGL((k_gemv_q<TT, NR, WGS>), dim3(grid), dim3(WGS), lds, s, (const uint8_t*)g.w, x,
-                     (uint8_t*)xq_out, g.out, g.rows, g.cols, g.row_bytes, upr, team, nullptr, nullptr, 0, 0L);
+  if (layout) {
+    if constexpr (act32(TT) && NR == 1 && WGS == 1024)
+      hipLaunchKernelGGL((k_gemv_q<TT, NR, WGS, false, true>), dim3(grid), dim3(WGS), lds, s, (const uint8_t*)g.w, x,
+                         (uint8_t*)xq_out, g.out, g.rows, g.cols, g.row_bytes, upr, team, nullptr, nullptr,
+                         layout >> 4, (long)(layout & 15));
+    else
+      return hipErrorInvalidValue;
+  } else {
+    hipLaunchKernelGGL((k_gemv_q<TT, NR, WGS>), dim3(grid), dim3(WGS), lds, s, (const uint8_t*)g.w, x,
+                       (uint8_t*)xq_out, g.out, g.rows, g.cols, g.row_bytes, upr, team, nullptr, nullptr, 0, 0L);
+  }
   return hipGetLastError();
 }
 
 template <int TT>
-static hipError_t launch_gemv_q_type(const GemvArgs& g, const float* x, void* xq_out, int team, int nr, int wgs,
-                                     hipStream_t s) {
-  if (wgs == 1024 && nr == 1) return launch_gemv_q_t<TT, 1, 1024>(g, x, xq_out, team, s);
-  if (wgs == 1024 && nr == 2) return launch_gemv_q_t<TT, 2, 1024>(g, x, xq_out, team, s);
-  if (wgs == 512 && nr == 1) return launch_gemv_q_t<TT, 1, 512>(g, x, xq_out, team, s);
-  if (wgs == 512 && nr == 2) return launch_gemv_q_t<TT, 2, 512>(g, x, xq_out, team, s);
+static hipError_t launch_gemv_q_type(const GemvArgs& g, const float* x, void* xq_out, int layout, int team, int nr,
+                                     int wgs, hipStream_t s) {
+  if (wgs == 1024 && nr == 1) return launch_gemv_q_t<TT, 1, 1024>(g, x, xq_out, layout, team, s);
+  if (wgs == 1024 && nr == 2) return launch_gemv_q_t<TT, 2, 1024>(g, x, xq_out, layout, team, s);
+  if (wgs == 512 && nr == 1) return launch_gemv_q_t<TT, 1, 512>(g, x, xq_out, layout, team, s);
+  if (wgs == 512 && nr == 2) return launch_gemv_q_t<TT, 2, 512>(g, x, xq_out, layout, team, s);
   if (wgs != 256) return hipErrorInvalidValue;
   switch (nr) {
-    case 1: return launch_gemv_q_t<TT, 1, 256>(g, x, xq_out, team, s);
-    case 2: return launch_gemv_q_t<TT, 2, 256>(g, x, xq_out, team, s);
-    case 4: return launch_gemv_q_t<TT, 4, 256>(g, x, xq_out, team, s);
+    case 1: return launch_gemv_q_t<TT, 1, 256>(g, x, xq_out, layout, team, s);
+    case 2: return launch_gemv_q_t<TT, 2, 256>(g, x, xq_out, layout, team, s);
+    case 4: return launch_gemv_q_t<TT, 4, 256>(g, x, xq_out, layout, team, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1105,9 +1125,10 @@ bool gemv_fused_preferred(const GemvArgs& g) {
 }
 
 hipError_t launch_gemv_fused(const GemvArgs& g, const float* x, void* xq_out, int team, int nr, int wgs,
-                             hipStream_t s) {
+                             hipStream_t s, int layout) {
   if (g.rows <= 0) return hipSuccess;
   if (g.tokens != 1 || g.kimg || !gemv_fused_fits(g.ttype, g.cols)) return hipErrorInvalidValue;
+  if (layout && (!act32(g.ttype) || (layout >> 4) * (layout & 15) * 64 != g.cols)) return hipErrorInvalidValue;
   if (team <= 0 && nr <= 0 && wgs <= 0) {
     fused_default_shape(g, team, nr, wgs);
   } else {
@@ -1116,7 +1137,7 @@ hipError_t launch_gemv_fused(const GemvArgs& g, const float* x, void* xq_out, in
     if (team <= 0) team = gemv_pick_team((g.rows + nr - 1) / nr, g.cols, kGemvTargetWaves);
   }
   return dispatch_type(g.ttype, [&](auto tt) {
-    return launch_gemv_q_type<decltype(tt)::value>(g, x, xq_out, team, nr, wgs, s);
+    return launch_gemv_q_type<decltype(tt)::value>(g, x, xq_out, layout, team, nr, wgs, s);
   });
 }
 

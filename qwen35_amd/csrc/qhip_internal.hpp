@@ -50,8 +50,13 @@ bool gemv_fused_fits(int ttype, int cols);
 bool gemv_fused_preferred(const GemvArgs& g);
 bool gemv_fused_one_round(const GemvArgs& g);
 // team / nr / wgs (workgroup threads: 256, or 512 / 1024 with nr <= 2) 0 = pick
+// layout: of xq_out, 0 the reference rows, else gemv_image_layout's (32-value
+// formats in the default shape past 2^23 weights)
 hipError_t launch_gemv_fused(const GemvArgs& g, const float* x, void* xq_out, int team, int nr, int wgs,
-                             hipStream_t s);
+                             hipStream_t s, int layout = 0);
+// the checks of qhip_launch_quantize_mul_mat_vec, then that launch (api.hip)
+int quantize_mul_mat_vec(const void* d_w, const float* d_x, void* d_xq_out, float* d_out, int rows, int cols, int ttype,
+                         int layout, hipStream_t s);
 // Split-K quantize + GEMV for one token on long rows: slices of `slice`
 // values (a multiple of 256) per workgroup, partial sums in `work`
 // (gemv_splitk_work_bytes; its first kSkCountBytes must be zero before the

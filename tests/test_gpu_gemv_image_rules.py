@@ -60,9 +60,13 @@ def test_prepared_pair_is_captured_from_its_images(gpu, oracle, backend, tt, row
     assert backend.mem_placed() == placed  # nothing was left to build
 
 
-@pytest.mark.parametrize("tt", [po.TT_Q8_0, po.TT_IQ4_NL])
-def test_memo_and_unaligned_x_read_the_image(gpu, oracle, backend, tt):
-    rows, cols = 3300, 2560  # above 2^23 weights, where the one-launch form is the faster of the two
+@pytest.mark.parametrize("cols", [2560, 4096])
+@pytest.mark.parametrize("tt", [po.TT_Q8_0, po.TT_IQ4_NL, po.TT_Q4_0])
+def test_memo_and_unaligned_x_read_the_image(gpu, oracle, backend, tt, cols):
+    """Past 2^23 weights, where the one-launch form is the faster of the two: an x
+    that it does not take, and one it has quantized already, are multiplied from
+    the image."""
+    rows = 3300
     w = synth.make_weight(tt, rows, cols, seed=75, tag=tt)
     lin = backend.load_linear(tt, rows, cols, w)
     base = backend.mem_placed()
@@ -76,23 +80,40 @@ def test_memo_and_unaligned_x_read_the_image(gpu, oracle, backend, tt):
         xd.copy_(torch.from_numpy(x[0]))
         for memo in (False, True):
             backend.set_act_memo(memo)
-            for again in range(2):
+            for again in range(3):
                 out = torch.empty(rows, device=gpu)
                 backend.matvec(out, lin, xd)
                 outs[shift, memo, again] = out
     want = oracle.matvec(tt, w, x)[0]
     for out in outs.values():
         assert rel_l2(out.cpu().numpy(), want) < TOL
-    image = outs[1, False, 0]
-    for key, out in outs.items():
-        if key[0] == 1 or key[1]:
-            assert torch.equal(out, image), key
-    hits, misses = backend.act_stats()
-    assert (hits, misses) == (2, 2)  # per x, the second product reuses the first one's activation
-    backend.set_act_memo(False)
-    backend.set_gemv_images(False)
-    backend.matvec(image, lin, buf[1:1 + cols])
-    assert not torch.equal(image, outs[0, True, 0])  # the rows are summed in another order
+    fused, image = outs[0, False, 0], outs[1, False, 0]
+    # where a row's terms are summed in another order, the bits tell the two apart
+    assert cols == 4096 or not torch.equal(fused, image)
+    for (shift, memo, again), out in outs.items():
+        # the one-launch form leaves the activation in the image's own layout
+        from_image = shift == 1 or (memo and again > 0)
+        assert torch.equal(out, image if from_image else fused), (shift, memo, again)
+    assert backend.act_stats() == (4, 2)  # per x, the later products reuse the first one's activation
+
+
+def test_memo_one_launch_rows_for_a_weight_without_image(gpu, oracle, backend):
+    """Without an image the one-launch form leaves the reference rows, as for a
+    weight too small for one, and the two kinds of one x do not meet."""
+    tt, cols = po.TT_Q8_0, 2560
+    ws = [synth.make_weight(tt, rows, cols, seed=79, tag=rows) for rows in (3300, 500)]
+    large, small = (backend.load_linear(tt, w.reshape(-1, 2720).shape[0], cols, w) for w in ws)
+    assert backend.prepare_linear(large) == 0
+    x = synth.make_act(cols, 1, seed=80)
+    xd = torch.from_numpy(x[0]).to(gpu)
+    want = [oracle.matvec(tt, w, x)[0] for w in ws]
+    backend.set_act_memo(True)
+    for images in (True, False):
+        backend.set_gemv_images(images)
+        for lin, ref in ((large, 0), (large, 0), (small, 1), (small, 1), (large, 0), (large, 0), (small, 1)):
+            out = torch.empty(lin.rows, device=gpu)
+            backend.matvec(out, lin, xd)
+            assert rel_l2(out.cpu().numpy(), want[ref]) < TOL
 
 
 # one round of the one-launch form's workgroups | a little past it
