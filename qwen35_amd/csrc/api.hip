@@ -218,12 +218,21 @@ bool mmq_image_preferred(const GemvArgs& g) {
 // the planes, [20480, 2048] 36.4 / 39.8); Q6_K to 96 where all three tiles'
 // workgroups run at once ([2560, 12032] x 80 30.2 us / 36.1 from the planes and
 // the rows; [4096, 9728] 1.06 of it, [3584, 10240] 1.10) or the weight is not
-// too large ([5120, 8192] 34.5 / 37.3, [12288, 5120] 46.4 / 49.2, [16384, 2048]
+// too large ([5120, 8192] 34.5 / 37.3, [13312, 5120] 47.1 / 50.3, [16384, 2048]
 // 28.8 / 32.2; [10240, 8192] 59.9 / 57.0, [16384, 5120] 1.05, [24576, 2048]
-// 1.10, [16384, 1024] 1.08).
+// 1.10, [16384, 1024] 1.08), or the rows' launch has up to 5/4 tiles of 128 rows
+// and 64 tokens per CU ([17408, 4096] 52.3 / 61.0, [20480, 4096] 59.0 / 63.7,
+// [18432, 5120] 65.0 / 68.3, [16640, 1024] 20.7 / 24.9; [20480, 5120] 74.5 / 70.2,
+// [20480, 1536] 32.0 / 29.3);
+// not where that launch's tiles just about fill the CUs once ([14336, 4096] 46.7
+// / 44.3).
 static bool wd_q6k_three_tiles(const GemvArgs& g) {
   if (3L * ((g.rows + 31) / 32) <= cus()) return g.cols < 12288;
-  return g.cols <= 8192 && (long)g.rows * g.cols < (1L << 26) && g.rows <= (g.cols < 2048 ? 12288 : 20480);
+  const long n = (long)g.rows * g.cols, tiles = tiles_of(g, 128);
+  if (g.cols < 2048) return g.rows <= 12288 || (g.cols <= 1024 && tiles > cus() && 8 * tiles <= 9L * cus());
+  if (tiles > cus() && 4 * tiles <= 5L * cus()) return g.cols <= 5120 && n < 3L << 25;
+  if (g.cols >= 3072 && tiles <= cus() && 8 * tiles >= 7L * cus()) return false;
+  return g.cols <= 8192 && n < 17L << 22 && g.rows <= 20480;
 }
 bool wd_image_preferred(const GemvArgs& g) {
   if (g.ttype == TT_Q8_0)

@@ -224,7 +224,8 @@ def image_bytes(tt, rows, cols, planes):
 @pytest.mark.parametrize("tt,rows,cols,routes", [
     (po.TT_Q6_K, 1640, 5120, {96: "frag", 97: "planes"}),
     (po.TT_Q6_K, 2720, 8448, {96: "frag"}), (po.TT_Q6_K, 2752, 8448, {64: "frag", 65: "planes"}),
-    (po.TT_Q6_K, 16384, 1024, {65: "planes"}),
+    (po.TT_Q6_K, 16384, 1024, {65: "planes"}), (po.TT_Q6_K, 16640, 4096, {96: "frag", 97: "planes"}),
+    (po.TT_Q6_K, 20512, 2048, {65: "planes"}), (po.TT_Q6_K, 14336, 3072, {64: "frag", 65: "planes"}),
     (po.TT_Q5_K, 1640, 5120, {128: "frag", 129: "planes"}),
     # the tile MMQ in one full round | rows of few super-blocks in many rows
     (po.TT_Q5_K, 16384, 1024, {96: "frag", 97: None, 128: None, 129: "planes"}),
