@@ -3065,14 +3065,17 @@ static hipError_t launch_mmq_rk_nw(const GemvArgs& g, hipStream_t s) {
 // / 12.3, [12288, 3072] x 16 12.3 / 13.2 / 13.8; Q6_K [17408, 5120] x 16 26.6 /
 // 27.2 / 30.0, [5120, 5120] x 2 15.2 / 12.0 / 10.8, [8192, 2560] x 8 11.7 / 10.9 /
 // 9.7, [4096, 8192] x 8 21.2 / 15.1 / 15.6 and x 9 24.0 / 17.9 / 17.2 (Q4_K x 16
-// 18.8 / 13.8 / 14.1).
+// 18.8 / 13.8 / 14.1).  With the weights' decode of more bits the twelve waves'
+// gain ends sooner: [6144, 6144] with 8 / 12 Q4_K x 4 10.6 / 10.0, x 16 12.4 / 13.2,
+// Q5_K x 4 11.8 / 11.7, x 8 12.1 / 12.7.
 static int rk_waves(const GemvArgs& g) {
   const int cus0 = qhip_gpu_cu_count(), cus = cus0 > 0 ? cus0 : 256, nsb = g.cols / 256;
   const long wgs = (long)((g.rows + 31) / 32) * ((g.tokens + 31) / 32);
   if (wgs <= cus) {
     if (g.tokens <= 32 && nsb >= 36) return 12;
+    const int most = nsb <= 12 || g.ttype == TT_Q6_K ? 16 : g.ttype == TT_Q4_K ? 8 : 4;
     const bool fewer = (nsb + 11) / 12 < (nsb + 7) / 8 && (nsb <= 28 || (g.ttype == TT_Q6_K && g.tokens > 8));
-    return g.tokens <= 16 && fewer ? 12 : 8;
+    return g.tokens <= most && fewer ? 12 : 8;
   }
   const int most = nsb <= 12 && nsb % 8 == 4 ? 8 : 16;
   return wgs <= 2L * cus && g.tokens <= most ? 8 : 4;
